@@ -228,7 +228,7 @@ __global__ __launch_bounds__(256) void build_all_pairs_kernel(uint4 const* __res
     unsigned const lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
     unsigned const i0 = blockIdx.x * AP_PER_GROUP;
     if (cond.slots) {
-        if (!displacement_aborts(cond.slots, cond.keep_bits)) return;   // the whole workgroup
+        if (!displacement_aborts(displacement_word(cond.slots), cond.slots, cond.keep_bits)) return;   // the whole workgroup
         if (threadIdx.x < AP_PER_GROUP && i0 + threadIdx.x < n)
             cond.r0[i0 + threadIdx.x] = cond.pos[2 * size_t(i0 + threadIdx.x)];
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(cond.rebuilt, 1u);
@@ -287,110 +287,70 @@ __global__ __launch_bounds__(256) void build_all_pairs_kernel(uint4 const* __res
     }
 }
 
+// *word := max(*word, v); the atomic only where it would change a word that
+// others raise too (a stale read costs one more atomic)
+__device__ __forceinline__ void raise_to(uint32_t* word, uint32_t v) {
+    if (v > __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(word, v);
+}
+
+// the pair of stats words that this workgroup raises
+__device__ __forceinline__ uint32_t* stat_pair(uint32_t* stats) {
+    return stats + blockIdx.x % STAT_SLOTS * STAT_STRIDE;
+}
+
 // --- cell segments: 16-bit slots into the LDS-staged neighbourhood union ----
 
-// Byte offset of entry c of a lane from the workgroup's list base: H + 2048
-// (c / 16) + 32 lane + 2 (c % 16), with H (a multiple of 2048) the lane's
-// wave block row 0.  The counter q keeps it with the lane field (bits 5..10)
-// set to ones, q = H + 2048 (c / 16) + 0x7e0 + 2 (c % 16): adding 2 then
-// carries from the entry field straight into the block field, and one bit
-// field insert of the lane bits gives the address.
-constexpr uint32_t NB16_LANE_BITS = 0x7e0u;
+// Byte offset of entry c of a lane from the workgroup's list base: H + 1024
+// (c / 8) + 16 lane + 2 (c % 8), with H (a multiple of 1024) the lane's wave
+// group row 0.  The counter q keeps it with the lane field (bits 4..9) set to
+// ones, q = H + 1024 (c / 8) + 0x3f0 + 2 (c % 8): adding 2 then carries from
+// the entry field straight into the group field, and one bit field insert of
+// the lane bits gives the address.
+constexpr uint32_t NB16_LANE_BITS = 0x3f0u;
 
 struct nb16_state {
+    uint32_t lo, hi;        // PACK: the last four entries, oldest lowest
     uint4 ri;
     unsigned own, ti;
     unsigned q, q0, qmax;   // counter; its value at c = 0 and at c = cap - 1
-    unsigned lane32;        // 32 (lane % 64)
+    unsigned lane16;        // 16 (lane % 64)
     char* list;             // the workgroup's list base (uniform)
 };
 
 __device__ __forceinline__ unsigned nb16_count(nb16_state const& s) {
-    return (((s.q >> 11) - (s.q0 >> 11)) << 4) + ((s.q & 31u) >> 1);
+    return (((s.q >> 10) - (s.q0 >> 10)) << 3) + ((s.q & 15u) >> 1);
 }
 
-// 2-byte stores straight to the blocked list: a lane fills one 32-byte block
-// at a time and a wave's blocks share 2 KiB, so the lines are complete in L2
-// before they are written back (no staging buffer, hence more workgroups per
-// CU; gathering entries in LDS and storing whole blocks measured 6% slower).
-// Entries past the capacity overwrite the particle's last slot instead of
-// branching: the count still exceeds the capacity, and the caller rebuilds
-// larger lists.
+// PACK: four entries gather in two registers (two VALU instructions an entry)
+// and go out as one 8-byte store.  A lane fills one 16-byte group at a time and
+// a wave's groups share 1 KiB, so the lines are complete in L2 before they are
+// written back; but each lane's store is a request of its own to L2, and with
+// 2-byte stores the 84 million requests of a build at N = 2^20 are its bound
+// (128 channels, one request a cycle each: 0.3 ms; 350 us, 263 us packed).
+// The split build of small systems (below) starts at any entry and stores each
+// by itself: there the appends' latency counts (42 against 50 us at N = 16,000
+// with one lane per particle).
+// Entries past the capacity are counted and not stored (the caller rebuilds
+// larger lists).
+template <bool PACK>
 __device__ __forceinline__ void append16(nb16_state& s, unsigned entry) {
-    unsigned const qa = min(s.q, s.qmax);
-    unsigned const o = (s.lane32 & NB16_LANE_BITS) | (qa & ~NB16_LANE_BITS);
-    *reinterpret_cast<uint16_t*>(s.list + o) = uint16_t(entry);
+    char* const at = s.list + (s.lane16 | (s.q & ~NB16_LANE_BITS));
+    if (PACK) {
+        s.lo = __builtin_amdgcn_alignbit(s.hi, s.lo, 16);
+        s.hi = __builtin_amdgcn_alignbit(entry, s.hi, 16);
+        if ((s.q & 6u) == 6u && s.q <= s.qmax)   // the last entry of an aligned four
+            *reinterpret_cast<uint2*>(at - 6) = make_uint2(s.lo, s.hi);
+    } else {
+        if (s.q <= s.qmax) *reinterpret_cast<uint16_t*>(at) = uint16_t(entry);
+    }
     s.q = (s.q + 2u) | NB16_LANE_BITS;
 }
 
 // the list entry is the record's byte offset in the full-record union (16
 // bytes per record, the layout the force kernel stages)
 
-// non-cubic box: FP32 squared distance of the scaled fixed-point differences
-template <bool MULTI, bool SELF>
-__device__ __forceinline__ void test16(nb16_state& s, uint4 const rj, unsigned slot, neighbour_params const& p,
-                                       uint32_t const* s_rr, uint32_t rr0) {
-#pragma clang fp contract(off)
-    float const dx = float(int32_t(s.ri.x - rj.x)) * p.q[0];
-    float const dy = float(int32_t(s.ri.y - rj.y)) * p.q[1];
-    float const dz = float(int32_t(s.ri.z - rj.z)) * p.q[2];
-    float rr = dx * dx;
-    rr = rr + dy * dy;
-    rr = rr + dz * dz;
-    bool const inside = rr <= __uint_as_float(MULTI ? s_rr[s.ti + (rj.w & 3u)] : rr0);
-    if ((!SELF || slot != s.own) && inside) append16(s, slot * 16u);
-}
-
-// cubic box, packed records: exact integer squared distance of the 16-bit
-// differences of the top halves (wrapped, hence the minimum image), at most
-// 3 * 2^30 and compared unsigned; s.ri.x and s.ri.y hold the particle's own
-// packed record
 typedef short short2v __attribute__((ext_vector_type(2)));
 typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
-template <bool MULTI, bool SELF>
-__device__ __forceinline__ void test16p(nb16_state& s, uint2 const rj, unsigned slot, uint32_t const* s_rr,
-                                        uint32_t rr0) {
-    ushort2v const dxy = __builtin_bit_cast(ushort2v, s.ri.x) - __builtin_bit_cast(ushort2v, rj.x);
-    int const dz = short(s.ri.y - rj.y);
-    short2v const d = __builtin_bit_cast(short2v, dxy);
-    uint32_t const rq = uint32_t(__builtin_amdgcn_sdot2(d, d, dz * dz, false));
-    bool const inside = rq <= (MULTI ? s_rr[s.ti + (rj.y >> 16)] : rr0);
-    if ((!SELF || slot != s.own) && inside) append16(s, slot * 16u);
-}
-
-// the 16-bit predicate of test16p alone
-template <bool MULTI>
-__device__ __forceinline__ bool pass16(nb16_state const& s, uint2 const rj, uint32_t const* s_rr, uint32_t rr0) {
-    ushort2v const dxy = __builtin_bit_cast(ushort2v, s.ri.x) - __builtin_bit_cast(ushort2v, rj.x);
-    int const dz = short(s.ri.y - rj.y);
-    short2v const d = __builtin_bit_cast(short2v, dxy);
-    uint32_t const rq = uint32_t(__builtin_amdgcn_sdot2(d, d, dz * dz, false));
-    return rq <= (MULTI ? s_rr[s.ti + (rj.y >> 16)] : rr0);
-}
-
-// candidates [t, e) of one row, four records in flight
-template <bool MULTI, bool SELF>
-__device__ __forceinline__ void scan16(nb16_state& s, unsigned t, unsigned const e, uint4 const* s_rec,
-                                       neighbour_params const& p, uint32_t const* s_rr, uint32_t rr0) {
-    for (; t + 4 <= e; t += 4) {
-        uint4 const r0 = s_rec[t], r1 = s_rec[t + 1], r2 = s_rec[t + 2], r3 = s_rec[t + 3];
-        test16<MULTI, SELF>(s, r0, t, p, s_rr, rr0);
-        test16<MULTI, SELF>(s, r1, t + 1, p, s_rr, rr0);
-        test16<MULTI, SELF>(s, r2, t + 2, p, s_rr, rr0);
-        test16<MULTI, SELF>(s, r3, t + 3, p, s_rr, rr0);
-    }
-    for (; t < e; ++t) test16<MULTI, SELF>(s, s_rec[t], t, p, s_rr, rr0);
-}
-// cubic box, packed records: the hits of up to 32 candidates gathered in a
-// bit mask with no branch, then appended in ascending candidate order: one
-// store instruction per round of the wave's remaining hits instead of one per
-// candidate.  Each candidate costs its test and one v_addc_co_u32 (m = 2 m +
-// the lane's bit of the compare's lane mask, the mask as carry-in).
-// Candidates go in groups of 4; a group may read up to 3 records past the
-// row's end (the launches give every workgroup at least 4 records of LDS past
-// its staging, the sentinel's slot and the cell-start table after it
-// included), whose bits one mask per chunk clears, as it clears the
-// particle's own bit.
 
 // m = 2 m + (this lane's bit of lanes)
 __device__ __forceinline__ uint32_t shift_in(uint32_t m, uint64_t lanes) {
@@ -400,67 +360,127 @@ __device__ __forceinline__ uint32_t shift_in(uint32_t m, uint64_t lanes) {
     return r;
 }
 
-// the lanes whose candidate rj passes the test of pass16 (compare lane mask)
-template <bool MULTI>
-__device__ __forceinline__ uint64_t pass16_lanes(nb16_state const& s, uint2 const rj, uint32_t const* s_rr,
-                                                 uint32_t rr0) {
+// cubic box, packed records: exact integer squared distance of the 16-bit
+// differences of the top halves (wrapped, hence the minimum image), at most
+// 3 * 2^30 and compared unsigned; s.ri.x and s.ri.y hold the particle's own
+// packed record
+__device__ __forceinline__ uint32_t square16(nb16_state const& s, uint2 const rj, int add) {
     ushort2v const dxy = __builtin_bit_cast(ushort2v, s.ri.x) - __builtin_bit_cast(ushort2v, rj.x);
     int const dz = short(s.ri.y - rj.y);
     short2v const d = __builtin_bit_cast(short2v, dxy);
-    uint32_t const rq = uint32_t(__builtin_amdgcn_sdot2(d, d, dz * dz, false));
-    uint32_t const thr = MULTI ? s_rr[s.ti + (rj.y >> 16)] : rr0;
-    return __builtin_amdgcn_uicmp(rq, thr, 37);   // 37: unsigned less or equal
+    return uint32_t(__builtin_amdgcn_sdot2(d, d, dz * dz + add, false));
+}
+// the predicate alone
+template <bool MULTI>
+__device__ __forceinline__ bool pass16(nb16_state const& s, uint2 const rj, uint32_t const* s_rr, uint32_t rr0) {
+    return square16(s, rj, 0) <= (MULTI ? s_rr[s.ti + (rj.y >> 16)] : rr0);
 }
 
-template <bool MULTI, bool SELF>
-__device__ __forceinline__ void scan16(nb16_state& s, unsigned t, unsigned const e, uint2 const* s_rec,
-                                       neighbour_params const&, uint32_t const* s_rr, uint32_t rr0) {
-    while (t < e) {
-        unsigned const n = min(e - t, 32u);
-        uint32_t m = 0;
-        unsigned k = 0;
-        for (; k < n; k += 4) {
-            uint2 const r0 = s_rec[t + k], r1 = s_rec[t + k + 1], r2 = s_rec[t + k + 2], r3 = s_rec[t + k + 3];
-            m = shift_in(m, pass16_lanes<MULTI>(s, r0, s_rr, rr0));
-            m = shift_in(m, pass16_lanes<MULTI>(s, r1, s_rr, rr0));
-            m = shift_in(m, pass16_lanes<MULTI>(s, r2, s_rr, rr0));
-            m = shift_in(m, pass16_lanes<MULTI>(s, r3, s_rr, rr0));
-        }
-        // k (n rounded up to whole groups) bits shifted in: candidate t + c
-        // at bit k - 1 - c, reversed at bit 32 - k + c = c - base (mod 2^32)
-        m = __builtin_bitreverse32(m);
-        unsigned const base = t + k - 32u;
-        m &= ~0u >> (k - n);   // candidates t + n .. t + k - 1 (k - n <= 3)
-        if (SELF) {
-            unsigned const ob = s.own - base;   // below 32 only inside the chunk or its empty low bits
-            m &= ob < 32u ? ~(1u << ob) : ~0u;
-        }
-        while (m) {
-            append16(s, (base + unsigned(__builtin_ctz(m))) * 16u);
-            m &= m - 1u;
-        }
-        t += n;
+// m = 2 m + 1 if the candidate is a neighbour, 2 m otherwise.
+// FOLD (one species, 5 or more cells a side): no coordinate difference of a
+// window exceeds 2/5 of the box, so that the squared distance less rr16 + 1 is
+// a signed 32-bit number whose sign is the test: five VALU instructions a
+// candidate instead of six (compare, carry-in).
+template <bool MULTI, bool FOLD>
+__device__ __forceinline__ uint32_t test_in(uint32_t m, nb16_state const& s, uint2 const rj,
+                                            neighbour_params const&, uint32_t const* s_rr, uint32_t rr0) {
+    if (FOLD) return __builtin_amdgcn_alignbit(m, square16(s, rj, -int(rr0) - 1), 31);
+    uint32_t const thr = MULTI ? s_rr[s.ti + (rj.y >> 16)] : rr0;
+    return shift_in(m, __builtin_amdgcn_uicmp(square16(s, rj, 0), thr, 37));   // 37: unsigned less or equal
+}
+// non-cubic box: FP32 squared distance of the scaled fixed-point differences
+template <bool MULTI, bool FOLD>
+__device__ __forceinline__ uint32_t test_in(uint32_t m, nb16_state const& s, uint4 const rj,
+                                            neighbour_params const& p, uint32_t const* s_rr, uint32_t rr0) {
+#pragma clang fp contract(off)
+    float const dx = float(int32_t(s.ri.x - rj.x)) * p.q[0];
+    float const dy = float(int32_t(s.ri.y - rj.y)) * p.q[1];
+    float const dz = float(int32_t(s.ri.z - rj.z)) * p.q[2];
+    float rr = dx * dx;
+    rr = rr + dy * dy;
+    rr = rr + dz * dz;
+    float const thr = __uint_as_float(MULTI ? s_rr[s.ti + (rj.w & 3u)] : rr0);
+    return shift_in(m, __builtin_amdgcn_fcmpf(rr, thr, 5));   // 5: ordered less or equal
+}
+
+// the hits of the n (1 .. 32) candidates from slot t, candidate c at bit 31 - c,
+// gathered with no branch.  Candidates go in groups of 4; a group may read up
+// to 3 records past the row's end (the launches give every workgroup at least
+// 4 records of LDS past its staging, the sentinel's slot and the cell-start
+// table after it included), whose bits the mask clears, as it clears the
+// particle's own bit.
+template <bool MULTI, bool FOLD, bool SELF, class Rec>
+__device__ __forceinline__ uint32_t scan_mask(nb16_state const& s, unsigned t, unsigned n, Rec const* s_rec,
+                                              neighbour_params const& p, uint32_t const* s_rr, uint32_t rr0) {
+    uint32_t m = 0;
+    unsigned k = 0;
+    for (; k < n; k += 4) {
+        Rec const r0 = s_rec[t + k], r1 = s_rec[t + k + 1], r2 = s_rec[t + k + 2], r3 = s_rec[t + k + 3];
+        m = test_in<MULTI, FOLD>(m, s, r0, p, s_rr, rr0);
+        m = test_in<MULTI, FOLD>(m, s, r1, p, s_rr, rr0);
+        m = test_in<MULTI, FOLD>(m, s, r2, p, s_rr, rr0);
+        m = test_in<MULTI, FOLD>(m, s, r3, p, s_rr, rr0);
+    }
+    m <<= 32u - k;
+    m &= uint32_t(int32_t(0x80000000u) >> (n - 1u));
+    if (SELF) {
+        unsigned const o = s.own - t;
+        m &= o < 32u ? ~(0x80000000u >> o) : ~0u;
+    }
+    return m;
+}
+
+// calls f(entry) for each hit in ascending candidate order, one round of the
+// wave per remaining hit of its lanes; entry0: the entry of candidate 0
+template <class F>
+__device__ __forceinline__ void each_hit(uint32_t m, unsigned entry0, F&& f) {
+    while (m) {
+        unsigned const c = unsigned(__builtin_clz(m));
+        m &= 0x7fffffffu >> c;
+        f(entry0 + c * 16u);
     }
 }
 
 // One cell segment of the staged list build (the whole workgroup calls it);
 // shared by the single-system kernel and the ensemble kernel.  The union is
 // staged as packed 16-bit records in a cubic box (8 bytes per record of the
-// dynamic LDS), else as full records (16 bytes).  stats[0] receives the
-// largest count, stats[1] the staging size U + 1.
-template <bool MULTI, bool ISO>
+// dynamic LDS), else as full records (16 bytes).  stats (optional): stats[0]
+// receives the largest count, stats[1] the staging size U + 1.
+//
+// SPLIT = 0: one lane per particle, its nine candidate rows in turn.
+// SPLIT > 0 (a workgroup of SPLIT times three waves): three waves take 64
+// particles together, one z-plane of candidate rows each.  They keep the hit
+// masks of their rows in LDS, and append them after those of the planes below,
+// whose counts the others have left there.  The tests of a lane are one chain
+// of dependent LDS reads, 47 us long at 0.84 particles per sigma^3 however few
+// particles there are; where waves are few, thirds of it side by side are
+// faster (27 us at N = 4000 and 16,000, 46 against 57 us at N = 64,000).
+constexpr unsigned SPLIT_WAVES = 3, SPLIT_MASKS = 9;   // masks a lane keeps; a later one is formed again
+template <unsigned SPLIT>
+struct build_stage {
+    uint32_t mask[SPLIT * SPLIT_WAVES][SPLIT_MASKS][WAVE];
+    uint32_t hits[SPLIT * SPLIT_WAVES][WAVE];
+};
+template <>
+struct build_stage<0> {};
+// a workgroup's LDS, and what the static tables take of it
+constexpr size_t BUILD_LDS_MAX = 64 << 10, BUILD_TABLES = sizeof(seg_stage) + MAX_TYPES * MAX_TYPES * 4 + 512;
+constexpr size_t ENS_BUILD_TABLES = BUILD_TABLES + SEG_NR * SEG_BOUND * 4;
+
+template <bool MULTI, bool ISO, bool FOLD, unsigned SPLIT>
 __device__ __forceinline__ void staged_build_segment(
     uint4 const* __restrict__ posq, uint32_t const* __restrict__ off, seg_params const& sp, unsigned seg,
     neighbour_params const& p, unsigned cap, uint16_t* __restrict__ list, uint32_t* __restrict__ count,
     uint32_t* __restrict__ stats, uint4* s_lds, seg_stage& st, unsigned* s_bound, uint32_t* s_rr,
-    unsigned bstride = SEG_BOUND, uint32_t* overflow = nullptr)
+    unsigned bstride, uint32_t* overflow, build_stage<SPLIT>& sh)
 {
+    static_assert(!(FOLD && (MULTI || !ISO)), "");
     using rec_t = typename std::conditional<ISO, uint2, uint4>::type;
     rec_t* const s_rec = reinterpret_cast<rec_t*>(s_lds);
     if (threadIdx.x < MAX_TYPES * MAX_TYPES)
         s_rr[threadIdx.x] = ISO ? p.rr16[threadIdx.x] : __float_as_uint(p.rr_cut_skin[threadIdx.x]);
-    unsigned const U = stage_union(sp, seg, off, posq, s_rec, st, s_bound, bstride);
-    if (threadIdx.x == 0) atomicMax(&stats[1], U + 1);
+    unsigned const U = stage_union(sp, seg, off, posq, s_rec, st, s_bound, bstride, [] { return false; });
+    if (stats && threadIdx.x == 0) raise_to(&stats[1], U + 1);
     if (U + 1 > sp.lds_cap) {   // uniform: the caller enlarges the staging and rebuilds
         if (overflow && threadIdx.x == 0) atomicOr(overflow, ENS_SKIP_OVERFLOW);
         return;
@@ -475,12 +495,20 @@ __device__ __forceinline__ void staged_build_segment(
     unsigned const i0 = st.own_begin[0] & ~(WAVE - 1);
     char* const wlist = reinterpret_cast<char*>(list + size_t(i0) * cap);
     unsigned cmax = 0;
-    for (unsigned t = threadIdx.x; t < T; t += blockDim.x) {
+    // SPLIT: wave w takes plane w % 3 of the particles of waves w / 3; every
+    // wave runs the same number of passes (they meet at barriers)
+    unsigned const lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    unsigned const plane = wave % SPLIT_WAVES, w0 = wave - plane;
+    for (unsigned t0 = 0; t0 < T; t0 += SPLIT ? SPLIT * WAVE : blockDim.x) {
+        unsigned const t = t0 + (SPLIT ? w0 / SPLIT_WAVES * WAVE + lane : threadIdx.x);
+        bool const live = t < T;
+        if (!SPLIT && !live) break;
         unsigned j, i;
-        seg_own(st, t, j, i);
+        seg_own(st, live ? t : 0u, j, i);
         unsigned const self = hh + j + 1;   // union row of the particle's own (y, z) row
         nb16_state s;
-        s.own = s_bound[self * bstride + 1] + (t - st.own_pre[j]);
+        s.lo = s.hi = 0;
+        s.own = s_bound[self * bstride + 1] + ((live ? t : 0u) - st.own_pre[j]);
         uint4 const full = posq[i];          // = the staged record s.own, in full
         if (ISO) {
             uint2 const pk = pack_rec16(full);
@@ -489,38 +517,93 @@ __device__ __forceinline__ void staged_build_segment(
             s.ri = full;
         }
         s.ti = (full.w & 3u) * p.ntype;
-        unsigned const H = 2 * ((i & ~(WAVE - 1)) - i0) * cap;   // multiple of 2048
+        unsigned const H = 2 * ((i & ~(WAVE - 1)) - i0) * cap;   // multiple of 1024
         s.q0 = H | NB16_LANE_BITS;
         s.q = s.q0;
-        s.qmax = s.q0 + (((cap - 1) >> 4) << 11) + (((cap - 1) & 15u) << 1);
-        s.lane32 = (i & (WAVE - 1)) * (2 * NB16_BLOCK);
+        s.qmax = s.q0 + (((cap - 1) >> 3) << 10) + (((cap - 1) & 7u) << 1);
+        s.lane16 = (i & (WAVE - 1)) * (2 * NB16_GROUP);
         s.list = wlist;
         unsigned const k = cell_component(full.x, nx) - st.q.x0;   // 0 .. w - 1
-        // the 9 rows (dz, dy) in lexicographic order; only the own row holds
-        // the particle itself
-        for (unsigned dz = 0; dz < 3; ++dz)
-            for (unsigned dy = 0; dy < 3; ++dy) {
-                unsigned const ur = dz * hh + j + dy;
-                unsigned const b = s_bound[ur * bstride + k];
-                unsigned const e = s_bound[ur * bstride + k + 3];
-                if (ur == self)
-                    scan16<MULTI, true>(s, b, e, s_rec, p, s_rr, rr0);
-                else
-                    scan16<MULTI, false>(s, b, e, s_rec, p, s_rr, rr0);
+        // the candidates of one row in chunks of 32: f(slot, candidates, whether
+        // the row is the particle's own)
+        auto row = [&](unsigned ur, auto&& f) {
+            unsigned b = s_bound[ur * bstride + k];
+            unsigned const e = s_bound[ur * bstride + k + 3];
+            for (; b < e; b += 32) f(b, min(e - b, 32u));
+        };
+        auto mask_of = [&](bool own_row, unsigned b, unsigned n) {
+            return own_row ? scan_mask<MULTI, FOLD, true>(s, b, n, s_rec, p, s_rr, rr0)
+                           : scan_mask<MULTI, FOLD, false>(s, b, n, s_rec, p, s_rr, rr0);
+        };
+        if constexpr (SPLIT > 0) {
+            unsigned hits = 0, c = 0;
+            if (live)
+                for (unsigned dy = 0; dy < 3; ++dy) {
+                    unsigned const ur = plane * hh + j + dy;
+                    row(ur, [&](unsigned b, unsigned n) {
+                        uint32_t const m = mask_of(ur == self, b, n);
+                        if (c < SPLIT_MASKS) sh.mask[wave][c][lane] = m;
+                        ++c;
+                        hits += unsigned(__builtin_popcount(m));
+                    });
+                }
+            sh.hits[wave][lane] = hits;
+            __syncthreads();
+            unsigned first = 0, total = 0;
+            for (unsigned w = 0; w < SPLIT_WAVES; ++w) {
+                unsigned const v = sh.hits[w0 + w][lane];
+                first += w < plane ? v : 0u;
+                total += v;
             }
-        unsigned const c = nb16_count(s);
-        // pad with the sentinel to a multiple of 8 (cap is a multiple of 16)
-        if (c <= cap)
-            while (s.q & 15u) append16(s, U * 16u);
-        count[i] = c;
-        cmax = max(cmax, c);
+            if (live) {
+                // the counter at entry `first`
+                s.q = s.q0 + ((first >> 3) << 10) + ((first & 7u) << 1);
+                c = 0;
+                for (unsigned dy = 0; dy < 3; ++dy) {
+                    unsigned const ur = plane * hh + j + dy;
+                    row(ur, [&](unsigned b, unsigned n) {
+                        uint32_t const m = c < SPLIT_MASKS ? sh.mask[wave][c][lane] : mask_of(ur == self, b, n);
+                        ++c;
+                        each_hit(m, b * 16u, [&](unsigned entry) { append16<false>(s, entry); });
+                    });
+                }
+                if (plane == SPLIT_WAVES - 1) {
+                    // pad with the sentinel to a multiple of 8 (cap is a multiple of 16)
+                    if (total <= cap)
+                        while (s.q & 15u) append16<false>(s, U * 16u);
+                    count[i] = total;
+                    cmax = max(cmax, total);
+                }
+            }
+            __syncthreads();   // the next pass reuses the masks
+        } else {
+            // the 9 rows (dz, dy) in lexicographic order; only the own row holds
+            // the particle itself
+            auto take = [&](uint32_t m, unsigned b) {
+                each_hit(m, b * 16u, [&](unsigned entry) { append16<true>(s, entry); });
+            };
+            for (unsigned dz = 0; dz < 3; ++dz)
+                for (unsigned dy = 0; dy < 3; ++dy) {
+                    unsigned const ur = dz * hh + j + dy;
+                    if (ur == self)
+                        row(ur, [&](unsigned b, unsigned n) { take(mask_of(true, b, n), b); });
+                    else
+                        row(ur, [&](unsigned b, unsigned n) { take(mask_of(false, b, n), b); });
+                }
+            unsigned const c = nb16_count(s);
+            // pad with the sentinel to a multiple of 8 (cap is a multiple of 16)
+            if (c <= cap)
+                while (s.q & 15u) append16<true>(s, U * 16u);
+            count[i] = c;
+            cmax = max(cmax, c);
+        }
     }
-    for (int o = WAVE / 2; o > 0; o >>= 1) cmax = max(cmax, (unsigned)__shfl_xor((int)cmax, o, WAVE));
-    if ((threadIdx.x % WAVE) == 0 && cmax > 0) atomicMax(&stats[0], cmax);
-    if (overflow && (threadIdx.x % WAVE) == 0 && cmax > cap) atomicOr(overflow, ENS_SKIP_OVERFLOW);
+    cmax = wave_max_u32(cmax);
+    if (stats && lane == 0) raise_to(&stats[0], cmax);
+    if (overflow && lane == 0 && cmax > cap) atomicOr(overflow, ENS_SKIP_OVERFLOW);
 }
 
-template <bool MULTI, bool ISO>
+template <bool MULTI, bool ISO, bool FOLD, unsigned SPLIT>
 __global__ __launch_bounds__(SEG_THREADS_MAX) void build_staged_kernel(
     uint4 const* __restrict__ posq, uint32_t const* __restrict__ off, seg_params sp, neighbour_params p,
     unsigned cap, uint16_t* __restrict__ list, uint32_t* __restrict__ count, uint32_t* __restrict__ stats)
@@ -528,6 +611,7 @@ __global__ __launch_bounds__(SEG_THREADS_MAX) void build_staged_kernel(
     extern __shared__ uint4 s_rec[];
     __shared__ seg_stage st;
     __shared__ uint32_t s_rr[MAX_TYPES * MAX_TYPES];
+    __shared__ build_stage<SPLIT> sh;
 
     unsigned const seg = seg_of_block(sp, blockIdx.x);
     if (seg >= sp.nseg) return;   // the whole workgroup
@@ -535,8 +619,8 @@ __global__ __launch_bounds__(SEG_THREADS_MAX) void build_staged_kernel(
     // (3 (R + 2) rows of S + 3 words), sized to the segment shape
     unsigned* const s_bound = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(s_rec) +
                                                           size_t(sp.lds_cap) * (ISO ? sizeof(uint2) : sizeof(uint4)));
-    staged_build_segment<MULTI, ISO>(posq, off, sp, seg, p, cap, list, count, stats, s_rec, st, s_bound, s_rr,
-                                     sp.S + 3);
+    staged_build_segment<MULTI, ISO, FOLD, SPLIT>(posq, off, sp, seg, p, cap, list, count, stat_pair(stats), s_rec, st,
+                                                 s_bound, s_rr, sp.S + 3, nullptr, sh);
 }
 
 // --- cell segments with x sub-bins: per-particle candidate windows ---------
@@ -570,8 +654,8 @@ __device__ __forceinline__ void windowed_build_segment(
 {
     uint2* const s_rec = reinterpret_cast<uint2*>(s_lds);
     if (threadIdx.x < MAX_TYPES * MAX_TYPES) s_rr[threadIdx.x] = p.rr16[threadIdx.x];
-    unsigned const U = stage_union(sp, seg, off, posq, s_rec, st, s_bound);
-    if (threadIdx.x == 0) atomicMax(&stats[1], U + 1);
+    unsigned const U = stage_union(sp, seg, off, posq, s_rec, st, s_bound, SEG_BOUND, [] { return false; });
+    if (stats && threadIdx.x == 0) raise_to(&stats[1], U + 1);
     if (U + 1 > sp.lds_cap) return;   // uniform: the caller enlarges the staging and rebuilds
 
     seg_place const q = st.q;
@@ -620,8 +704,8 @@ __device__ __forceinline__ void windowed_build_segment(
         unsigned const H = 2 * ((i & ~(WAVE - 1)) - i0) * cap;
         s.q0 = H | NB16_LANE_BITS;
         s.q = s.q0;
-        s.qmax = s.q0 + (((cap - 1) >> 4) << 11) + (((cap - 1) & 15u) << 1);
-        s.lane32 = (i & (WAVE - 1)) * (2 * NB16_BLOCK);
+        s.qmax = s.q0 + (((cap - 1) >> 3) << 10) + (((cap - 1) & 7u) << 1);
+        s.lane16 = (i & (WAVE - 1)) * (2 * NB16_GROUP);
         s.list = wlist;
 
         uint32_t rrmax = rr0;
@@ -673,10 +757,10 @@ __device__ __forceinline__ void windowed_build_segment(
             bool const h1 = pass16<MULTI>(s, a1, s_rr, rr0) && c0 + 1 < ce;
             bool const h2 = pass16<MULTI>(s, a2, s_rr, rr0) && c0 + 2 < ce;
             bool const h3 = pass16<MULTI>(s, a3, s_rr, rr0) && c0 + 3 < ce;
-            if (h0) append16(s, c0 * 16u);
-            if (h1) append16(s, c0 * 16u + 16u);
-            if (h2) append16(s, c0 * 16u + 32u);
-            if (h3) append16(s, c0 * 16u + 48u);
+            if (h0) append16<false>(s, c0 * 16u);
+            if (h1) append16<false>(s, c0 * 16u + 16u);
+            if (h2) append16<false>(s, c0 * 16u + 32u);
+            if (h3) append16<false>(s, c0 * 16u + 48u);
             c0 += 4;
             if (c0 >= ce) {
                 ++r;
@@ -687,12 +771,12 @@ __device__ __forceinline__ void windowed_build_segment(
         }
         unsigned const c = nb16_count(s);
         if (c <= cap)
-            while (s.q & 15u) append16(s, U * 16u);
+            while (s.q & 15u) append16<false>(s, U * 16u);
         count[i] = c;
         cmax = max(cmax, c);
     }
-    for (int o = WAVE / 2; o > 0; o >>= 1) cmax = max(cmax, (unsigned)__shfl_xor((int)cmax, o, WAVE));
-    if ((threadIdx.x % WAVE) == 0 && cmax > 0) atomicMax(&stats[0], cmax);
+    cmax = wave_max_u32(cmax);
+    if (stats && (threadIdx.x % WAVE) == 0) raise_to(&stats[0], cmax);
 }
 
 template <bool MULTI>
@@ -709,7 +793,7 @@ __global__ __launch_bounds__(SEG_THREADS_MAX) void build_windowed_kernel(
 
     unsigned const seg = seg_of_block(sp, blockIdx.x);
     if (seg >= sp.nseg) return;   // the whole workgroup
-    windowed_build_segment<MULTI>(posq, off, soff, sp, seg, p, cap, list, count, stats, s_rec, st, s_bound, s_rr,
+    windowed_build_segment<MULTI>(posq, off, soff, sp, seg, p, cap, list, count, stat_pair(stats), s_rec, st, s_bound, s_rr,
                                   s_yz);
 }
 
@@ -829,8 +913,10 @@ __global__ __launch_bounds__(SEG_THREADS_MAX) void ens_build_kernel(
     uint32_t const e = rseg[blockIdx.x];
     unsigned const sys = e >> 16, seg = e & 0xffffu;
     ens_desc const& d = descs[sys];
-    staged_build_segment<MULTI, true>(posq + d.base, offsets + d.cell_base, d.sp, seg, d.np, d.cap,
-                                      list + d.list_off, count + d.base, stats + 2 * sys, s_rec, st, s_bound, s_rr);
+    build_stage<0> none;
+    staged_build_segment<MULTI, true, false, 0>(posq + d.base, offsets + d.cell_base, d.sp, seg, d.np, d.cap,
+                                                list + d.list_off, count + d.base, stats + 2 * sys, s_rec, st, s_bound,
+                                                s_rr, SEG_BOUND, nullptr, none);
 }
 
 // all-pairs lists of small systems: the workgroup builds the lists of
@@ -1303,8 +1389,9 @@ __global__ __launch_bounds__(256) void ens_copyback_flagged_kernel(
 }
 
 // the staged list build over the flagged segments
-template <bool MULTI>
-__global__ __launch_bounds__(SEG_THREADS_MAX) void ens_build_flagged_kernel(
+constexpr unsigned ENS_BUILD_SPLIT = 4;   // 256 particles a pass: a segment's, most often
+template <bool MULTI, unsigned SPLIT>
+__global__ __launch_bounds__(SPLIT ? SPLIT * SPLIT_WAVES * WAVE : SEG_THREADS_MAX) void ens_build_flagged_kernel(
     uint4 const* __restrict__ posq, uint32_t const* __restrict__ offsets, ens_desc const* __restrict__ descs,
     uint32_t* skip, ens_work w, uint16_t* __restrict__ list, uint32_t* __restrict__ count,
     uint32_t* __restrict__ stats)
@@ -1313,6 +1400,7 @@ __global__ __launch_bounds__(SEG_THREADS_MAX) void ens_build_flagged_kernel(
     __shared__ seg_stage st;
     __shared__ unsigned s_bound[SEG_NR * SEG_BOUND];
     __shared__ uint32_t s_rr[MAX_TYPES * MAX_TYPES];
+    __shared__ build_stage<SPLIT> sh;
     __shared__ uint32_t s_skip;
     unsigned const nl = w.head[0];
     uint32_t const total = w.lseg[nl];
@@ -1326,9 +1414,9 @@ __global__ __launch_bounds__(SEG_THREADS_MAX) void ens_build_flagged_kernel(
         bool const skipped = s_skip != 0;
         if (!skipped) {
             ens_desc const& d = descs[s];
-            staged_build_segment<MULTI, true>(posq + d.base, offsets + d.cell_base, d.sp, g - w.lseg[k], d.np, d.cap,
-                                              list + d.list_off, count + d.base, stats + 2 * s, s_rec, st, s_bound,
-                                              s_rr, SEG_BOUND, &skip[s]);
+            staged_build_segment<MULTI, true, false, SPLIT>(
+                posq + d.base, offsets + d.cell_base, d.sp, g - w.lseg[k], d.np, d.cap, list + d.list_off,
+                count + d.base, nullptr, s_rec, st, s_bound, s_rr, SEG_BOUND, &skip[s], sh);
         }
         __syncthreads();   // the next segment reuses the LDS
     }
@@ -1402,7 +1490,7 @@ void launch_build_neighbours(uint4 const* posq, unsigned n, uint32_t const* offs
 
 namespace halmd {
 
-void launch_build_neighbours_staged(uint4 const* posq, uint32_t const* offset, seg_params const& sp,
+void launch_build_neighbours_staged(uint4 const* posq, unsigned n, uint32_t const* offset, seg_params const& sp,
                                     neighbour_params const& p, unsigned cap, uint16_t* list, uint32_t* count,
                                     uint32_t* stats, hipStream_t s, uint32_t const* sub_offset) {
     if (!sp.nseg) return;
@@ -1420,20 +1508,25 @@ void launch_build_neighbours_staged(uint4 const* posq, uint32_t const* offset, s
         HIP_CHECK(hipGetLastError());
         return;
     }
-    size_t const lds = size_t(sp.lds_cap) * (p.iso ? sizeof(uint2) : sizeof(uint4)) +
-                       size_t(3) * (sp.R + 2) * (sp.S + 3) * sizeof(unsigned);
+    size_t const bounds = size_t(3) * (sp.R + 2) * (sp.S + 3) * sizeof(unsigned);
+    size_t const lds = size_t(sp.lds_cap) * (p.iso ? sizeof(uint2) : sizeof(uint4)) + bounds;
+    bool const split = n < BUILD_SPLIT_BELOW && lds + sizeof(build_stage<1>) + BUILD_TABLES <= BUILD_LDS_MAX;
+    bool const fold = p.ntype == 1 && p.iso && std::min({sp.grid.ncell[0], sp.grid.ncell[1], sp.grid.ncell[2]}) >= 5;
+    auto const go = [&](auto kernel, unsigned threads) {
+        kernel<<<grid, threads, lds, s>>>(posq, offset, sp, p, cap, list, count, stats);
+    };
+#define HALMD_BUILD_STAGED(...)                                                                                       \
+    (split ? go(build_staged_kernel<__VA_ARGS__, 1>, SPLIT_WAVES * WAVE)                                           \
+           : go(build_staged_kernel<__VA_ARGS__, 0>, sp.threads))
     if (p.ntype > 1) {
-        if (p.iso)
-            build_staged_kernel<true, true><<<grid, sp.threads, lds, s>>>(posq, offset, sp, p, cap, list, count, stats);
-        else
-            build_staged_kernel<true, false><<<grid, sp.threads, lds, s>>>(posq, offset, sp, p, cap, list, count, stats);
+        if (p.iso) HALMD_BUILD_STAGED(true, true, false);
+        else HALMD_BUILD_STAGED(true, false, false);
     } else {
-        if (p.iso)
-            build_staged_kernel<false, true><<<grid, sp.threads, lds, s>>>(posq, offset, sp, p, cap, list, count, stats);
-        else
-            build_staged_kernel<false, false><<<grid, sp.threads, lds, s>>>(posq, offset, sp, p, cap, list, count,
-                                                                          stats);
+        if (fold) HALMD_BUILD_STAGED(false, true, true);
+        else if (p.iso) HALMD_BUILD_STAGED(false, true, false);
+        else HALMD_BUILD_STAGED(false, false, false);
     }
+#undef HALMD_BUILD_STAGED
     HIP_CHECK(hipGetLastError());
 }
 
@@ -1552,12 +1645,18 @@ void launch_ens_rebuild_device(ens_rebuild_args const& a, hipStream_t s) {
     if (a.lds_records) {
         // cubic boxes: packed records, and 4 records of slack for the scan's last group
         size_t const lds = (size_t(a.lds_records) + 4) * sizeof(uint2);
+        auto const go = [&](auto kernel, unsigned threads) {
+            kernel<<<ENS_WORK_GRID, threads, lds, s>>>(a.posq, a.offsets, a.descs, a.skip, a.w, a.list, a.count,
+                                                       a.stats);
+        };
+        constexpr unsigned T = ENS_BUILD_SPLIT * SPLIT_WAVES * WAVE;
+        bool const split = lds + sizeof(build_stage<ENS_BUILD_SPLIT>) + ENS_BUILD_TABLES <= BUILD_LDS_MAX;
         if (a.multi)
-            ens_build_flagged_kernel<true><<<ENS_WORK_GRID, a.threads, lds, s>>>(a.posq, a.offsets, a.descs, a.skip,
-                                                                                a.w, a.list, a.count, a.stats);
+            split ? go(ens_build_flagged_kernel<true, ENS_BUILD_SPLIT>, T)
+                  : go(ens_build_flagged_kernel<true, 0>, SEG_THREADS_MAX);
         else
-            ens_build_flagged_kernel<false><<<ENS_WORK_GRID, a.threads, lds, s>>>(a.posq, a.offsets, a.descs, a.skip,
-                                                                                 a.w, a.list, a.count, a.stats);
+            split ? go(ens_build_flagged_kernel<false, ENS_BUILD_SPLIT>, T)
+                  : go(ens_build_flagged_kernel<false, 0>, SEG_THREADS_MAX);
         HIP_CHECK(hipGetLastError());
     }
     if (a.small_max_n) {

@@ -219,9 +219,39 @@ __device__ __forceinline__ T wave_sum(T v) {
     return v;
 }
 
+// v from the lane that the DPP control names, `other` where there is none
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ uint32_t dpp(uint32_t other, uint32_t v) {
+    return uint32_t(__builtin_amdgcn_update_dpp(int(other), int(v), CTRL, ROWS, 0xf, false));
+}
+
+// The wave scans go up the lanes of each row of 16 (row shifts), then across
+// the rows (row broadcasts): seven VALU instructions, where shuffles through
+// LDS take six dependent LDS round trips.
+__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t x) {
+    x += dpp<0x111>(0u, x);        // row_shr 1
+    x += dpp<0x112>(0u, x);
+    x += dpp<0x114>(0u, x);
+    x += dpp<0x118>(0u, x);
+    x += dpp<0x142, 0xa>(0u, x);   // row_bcast 15 into rows 1 and 3
+    x += dpp<0x143, 0xc>(0u, x);   // row_bcast 31 into rows 2 and 3
+    return x;
+}
+
+// the largest value of the wave, in every lane
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
+    x = max(x, dpp<0x111>(0u, x));
+    x = max(x, dpp<0x112>(0u, x));
+    x = max(x, dpp<0x114>(0u, x));
+    x = max(x, dpp<0x118>(0u, x));
+    x = max(x, dpp<0x142, 0xa>(0u, x));
+    x = max(x, dpp<0x143, 0xc>(0u, x));
+    return uint32_t(__builtin_amdgcn_readlane(int(x), 63));
+}
+
+// the same for values >= 0 (NaN is passed over, as fmaxf does)
 __device__ __forceinline__ float wave_max(float v) {
-    for (int off = WAVE / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, WAVE));
-    return v;
+    return __uint_as_float(wave_max_u32(__float_as_uint(fmaxf(v, 0.0f))));
 }
 
 } // namespace halmd

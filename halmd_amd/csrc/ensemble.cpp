@@ -49,8 +49,7 @@ uint4 const* cu4(dbuf<T> const& b) { return reinterpret_cast<uint4 const*>(b.get
 } // namespace
 
 ensemble::ensemble() {
-    // particles per cell segment (one 256-thread workgroup of the list build
-    // and the force); HALMD_SEG_TARGET overrides, as for single systems
+    // particles per cell segment; HALMD_SEG_TARGET overrides, as for single systems
     if (char const* e = std::getenv("HALMD_SEG_TARGET")) seg_target_ = std::max(1.0, std::atof(e));
     // stretches replayed from hipGraphs on request (HALMD_ENSEMBLE_GRAPHS=1):
     // measured 3% slower than eager launches on the 256-system workload
@@ -184,7 +183,11 @@ void ensemble::prepare(sys_host& h) {
         double const occ = double(h.n) / h.ncells;
         cell_grid g;
         g.ncell[0] = g.ncell[1] = g.ncell[2] = h.ncell;
-        segment_shape(occ, g, seg_target_, h.S, h.R);
+        // about a workgroup's threads, of systems that fill the chip together;
+        // from FORCE_STREAMS_BELOW on a particle's sums follow the segments, and
+        // they are those of the system alone
+        double const target = seg_target_ > 0 ? seg_target_ : force_streams(h.n) ? 200.0 : segment_target(h.n);
+        segment_shape(occ, g, target, h.S, h.R);
         h.nsx = unsigned(div_up(h.ncell, h.S));
         h.nsy = unsigned(div_up(h.ncell, h.R));
         h.nseg = h.nsx * h.nsy * h.ncell;

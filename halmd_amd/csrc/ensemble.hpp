@@ -100,7 +100,7 @@ public:
 private:
     std::vector<std::unique_ptr<sys_host>> sys_;
     bool committed_ = false, pending_ = false, device_steps_ = true;
-    double seg_target_ = 200;
+    double seg_target_ = 0;   // 0: by the system's size
     uint64_t recoveries_ = 0;
     uint64_t next_uid_ = 1;
     unsigned total_ = 0, nblocks_ = 0, threads_ = SEG_THREADS_MAX;

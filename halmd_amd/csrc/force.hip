@@ -4,7 +4,7 @@
 // with the potentials lennard_jones / morse (potentials/pair/*_kernel.hpp) and
 // the truncations sharp / shifted / force_shifted / smooth_r4
 // (potentials/pair/truncations/*_kernel.cuh).  One thread per particle walks
-// its neighbour list (blocks of 16 entries per lane, contiguous over the wave)
+// its neighbour list (groups of entries per lane, contiguous over the wave)
 // and gathers the 16-byte fixed-point record of each neighbour.
 //
 // Precision: the separation is the exact integer difference of the fixed-point
@@ -356,15 +356,24 @@ __global__ __launch_bounds__(256) void pair_force_split_kernel(
 //    operations.
 //  - MULTI: pair parameters by species from LDS; otherwise the one parameter
 //    set lives in scalar registers.
-// Summation: FP32 over blocks of 16 pairs, Kahan over the blocks (force,
-// energy and stress alike).
-// Lanes: lane t % 64 of the wave that covers particles t - t % 64 .. + 63.  The
-// segment's last wave is mostly empty (its particle count mod 64), so there the
-// list of each of its `active` particles is split into k = 64 / active (at most
-// SPLIT_MAX) runs of whole 16-slot blocks, one lane each, and lane p adds the
-// runs of lanes p + active, p + 2 active, ... in that order (Kahan).  Both the
-// split and the order depend only on the segment's particle count, never on
-// the workgroup size.
+// How the sums of a particle are formed, by the system's particle count alone
+// (force_streams), so that a system's trajectory does not depend on what it
+// shares a launch with:
+//  - STREAMS: two streams, the even and the odd groups of 8 slots; FP32 over
+//    two groups of a stream, Kahan over these, then the two streams are added.
+//    A wave of at most 32 particles takes two lanes per particle, one stream
+//    each; a fuller one takes the streams in turn.  The sums depend neither on
+//    the segment shape nor on the workgroup size, so that the shape can follow
+//    the system's size: a system of some 10^4 particles takes segments of one
+//    or two cells (more workgroups), while in an ensemble that fills the chip
+//    it keeps large ones (less staging).
+//  - otherwise FP32 over blocks of two groups, Kahan over the blocks.  The
+//    segment's last wave is mostly empty (its particle count mod 64), so there
+//    the list of each of its `active` particles is split into k = 64 / active
+//    (at most SPLIT_MAX) runs of whole blocks, one lane each, and lane p adds
+//    the runs of lanes p + active, p + 2 active, ... in that order (Kahan).
+//    One pass over the list: at N = 2^20, where issue is the bound, 96 us
+//    against 103 us with streams (equal below 2^18).
 // One cell segment of the staged force: the whole workgroup calls it for the
 // segment `seg` of the system described by (posq, off, sp, list, count, cap,
 // P); shared by the single-system kernel and the ensemble kernel.
@@ -372,7 +381,7 @@ constexpr unsigned SPLIT_MAX = 8;
 
 // FUSE (no aux): each particle is integrated (fused_integrate) as soon as its
 // force is final, instead of having its force written.
-template <int KIND, int TRUNC, bool AUX, bool ISO, bool MULTI, bool FUSE = false>
+template <int KIND, int TRUNC, bool AUX, bool ISO, bool MULTI, bool FUSE, bool STREAMS>
 __device__ __forceinline__ float staged_force_segment(
     uint4 const* __restrict__ posq, uint32_t const* __restrict__ off, seg_params const& sp, unsigned seg,
     uint16_t const* __restrict__ list, uint32_t const* __restrict__ count, unsigned cap, force_params const& P,
@@ -385,7 +394,7 @@ __device__ __forceinline__ float staged_force_segment(
         ISO && KIND == POTENTIAL_LENNARD_JONES && (TRUNC == TRUNC_SHARP || TRUNC == TRUNC_SHIFTED);
     constexpr bool P0_OUT = LJQ && !MULTI;   // 48 eps / sigma^2 applied per particle
     if (MULTI && threadIdx.x < MAX_TYPES * MAX_TYPES) s_pair[threadIdx.x] = P.pair[threadIdx.x];
-    stage_union(sp, seg, off, posq, s_rec, st, nullptr);   // fits: the list build checked it
+    stage_union(sp, seg, off, posq, s_rec, st, nullptr, 0u, [] { return false; });   // fits: the list build checked it
 
     unsigned const T = st.own_pre[st.q.h];
     unsigned const lane = threadIdx.x % WAVE;
@@ -393,8 +402,9 @@ __device__ __forceinline__ float staged_force_segment(
     // cross-lane sums below need the whole wave)
     for (unsigned t0 = threadIdx.x - lane; t0 < T; t0 += blockDim.x) {
         unsigned const active = min(T - t0, WAVE);
-        unsigned const k = min(WAVE / active, SPLIT_MAX);   // lanes per particle: 1 in full waves
-        unsigned const part = lane / active;                // run of the list this lane takes
+        // lanes per particle (wave-uniform): 1 in full waves
+        unsigned const k = STREAMS ? (active <= WAVE / 2 ? 2u : 1u) : min(WAVE / active, SPLIT_MAX);
+        unsigned const part = lane / active;    // stream, or run of the list, that this lane takes
         unsigned const t = t0 + lane % active;
         bool const mine = part < k;
 
@@ -403,20 +413,19 @@ __device__ __forceinline__ float staged_force_segment(
         uint4 const qi = posq[i];
         unsigned const ti = (qi.w & 3u) * P.ntype;
         unsigned const n8 = (count[i] + 7u) & ~7u;
-        unsigned const nblk = (n8 + NB16_BLOCK - 1) / NB16_BLOCK;
-        unsigned const b_begin = mine ? nblk * part / k : 0u;
-        unsigned const b_end = mine ? nblk * (part + 1) / k : 0u;
         uint4 const* const lp =
-            reinterpret_cast<uint4 const*>(list + size_t(i & ~(WAVE - 1)) * cap + (i & (WAVE - 1)) * NB16_BLOCK);
+            reinterpret_cast<uint4 const*>(list + size_t(i & ~(WAVE - 1)) * cap) + (i & (WAVE - 1));
 
-        float fx = 0, fy = 0, fz = 0, cx = 0, cy = 0, cz = 0;
-        float bx = 0, by = 0, bz = 0;
-        float en = 0, s0 = 0, s1 = 0, s2 = 0, s3 = 0, s4 = 0, s5 = 0;   // per block of 16 pairs
-        float ka[7] = {}, kc[7] = {};   // aux sums over the blocks (Kahan)
+        // a stream's plain sums (16 pairs) and the Kahan sums over these: force,
+        // and with AUX energy and stress
+        constexpr int NS = AUX ? 10 : 3;
+        struct stream {
+            float b[NS] = {}, f[NS] = {}, c[NS] = {};
+        };
 
         // branch-free: most candidates lie inside the cutoff, so the wave
         // evaluates every pair and a select drops those beyond it
-        auto pair = [&](uint4 const qj) {
+        auto pair = [&](stream& a, uint4 const qj) {
             int32_t const Dx = int32_t(qi.x - qj.x), Dy = int32_t(qi.y - qj.y), Dz = int32_t(qi.z - qj.z);
             pair_param const& pp = MULTI ? s_pair[ti + (qj.w & 3u)] : P.pair[0];
             float dx, dy, dz, fval, u = 0.0f;
@@ -466,88 +475,105 @@ __device__ __forceinline__ float staged_force_segment(
                 pair_eval<KIND, TRUNC>(rr, md, pp, P.rri_smooth, fval, u);
             }
             fval = inside ? fval : 0.0f;
-            bx += fval * dx;
-            by += fval * dy;
-            bz += fval * dz;
-            if (AUX) {
-                en += inside ? u : 0.0f;
-                s0 += fval * dx * dx;
-                s1 += fval * dy * dy;
-                s2 += fval * dz * dz;
-                s3 += fval * dx * dy;
-                s4 += fval * dx * dz;
-                s5 += fval * dy * dz;
+            a.b[0] += fval * dx;
+            a.b[1] += fval * dy;
+            a.b[2] += fval * dz;
+            if constexpr (AUX) {
+                a.b[3] += inside ? u : 0.0f;
+                a.b[4] += fval * dx * dx;
+                a.b[5] += fval * dy * dy;
+                a.b[6] += fval * dz * dz;
+                a.b[7] += fval * dx * dy;
+                a.b[8] += fval * dx * dz;
+                a.b[9] += fval * dy * dz;
             }
         };
         // list entries are byte offsets of records in the staged union
         char const* const lds = reinterpret_cast<char const*>(s_rec);
         auto rec = [&](unsigned byte_off) { return *reinterpret_cast<uint4 const*>(lds + byte_off); };
-        auto group = [&](uint4 const w) {
+        auto group = [&](stream& a, uint4 const w) {
             uint4 const q0 = rec(w.x & 0xffffu), q1 = rec(w.x >> 16), q2 = rec(w.y & 0xffffu), q3 = rec(w.y >> 16),
                         q4 = rec(w.z & 0xffffu), q5 = rec(w.z >> 16), q6 = rec(w.w & 0xffffu), q7 = rec(w.w >> 16);
-            pair(q0); pair(q1); pair(q2); pair(q3);
-            pair(q4); pair(q5); pair(q6); pair(q7);
+            pair(a, q0); pair(a, q1); pair(a, q2); pair(a, q3);
+            pair(a, q4); pair(a, q5); pair(a, q6); pair(a, q7);
         };
-        auto fold = [&]() {
-            kahan_add(fx, cx, bx);
-            kahan_add(fy, cy, by);
-            kahan_add(fz, cz, bz);
-            bx = by = bz = 0;
-            if (AUX) {
-                float const blk[7] = {en, s0, s1, s2, s3, s4, s5};
+        auto fold = [&](stream& a) {
 #pragma unroll
-                for (int c = 0; c < 7; ++c) kahan_add(ka[c], kc[c], blk[c]);
-                en = s0 = s1 = s2 = s3 = s4 = s5 = 0;
+            for (int k = 0; k < NS; ++k) {
+                kahan_add(a.f[k], a.c[k], a.b[k]);
+                a.b[k] = 0;
             }
         };
-        // blocks of 16 slots (two uint4 = two groups); the next block is
-        // loaded while the current one is evaluated
-        constexpr size_t BLOCK_STRIDE = WAVE * NB16_BLOCK * 2 / 16;   // uint4 between blocks of a lane
-        // (unconditional loads, the block index clamped into this particle's
-        // cap / 16 blocks, so that the wait for block b does not also wait
-        // for the prefetch of block b + 1)
-        unsigned const last = cap / NB16_BLOCK - 1;
-        unsigned const bf = min(b_begin, last);
-        uint4 w0 = lp[bf * BLOCK_STRIDE], w1 = lp[bf * BLOCK_STRIDE + 1];
-        for (unsigned b = b_begin; b < b_end; ++b) {
-            unsigned const bn = min(b + 1, last);
-            uint4 const n0 = lp[bn * BLOCK_STRIDE], n1 = lp[bn * BLOCK_STRIDE + 1];
-            group(w0);
-            if (n8 - b * NB16_BLOCK > 8) group(w1);
-            fold();
-            w0 = n0;
-            w1 = n1;
-        }
-        float rx = fx - cx, ry = fy - cy, rz = fz - cz;
-        if (AUX) {
-            en = ka[0] - kc[0]; s0 = ka[1] - kc[1]; s1 = ka[2] - kc[2]; s2 = ka[3] - kc[3];
-            s3 = ka[4] - kc[4]; s4 = ka[5] - kc[5]; s5 = ka[6] - kc[6];
-        }
-        if (k > 1) {   // wave-uniform
-            // lane p (part 0) collects the runs of lanes p + active, ... in order
-            // (the shuffles read every lane's own run, never a running sum)
-            float sx = rx, sy = ry, sz = rz, ex = 0, ey = 0, ez = 0;
-            float const aux[7] = {en, s0, s1, s2, s3, s4, s5};
-            float acc[7] = {en, s0, s1, s2, s3, s4, s5};
-            for (unsigned m = 1; m < k; ++m) {
-                unsigned const src = lane + m * active;
-                int const sl = int(src < WAVE ? src : lane);
-                kahan_add(sx, ex, __shfl(rx, sl, WAVE));
-                kahan_add(sy, ey, __shfl(ry, sl, WAVE));
-                kahan_add(sz, ez, __shfl(rz, sl, WAVE));
-                if (AUX) {
-#pragma unroll
-                    for (int c = 0; c < 7; ++c) acc[c] += __shfl(aux[c], sl, WAVE);
+        // groups of 8 slots (one uint4); the next two are loaded while two are
+        // evaluated (unconditional loads, the group index clamped into this
+        // particle's cap / 8 groups, so that the wait for a group does not also
+        // wait for the prefetch of the next)
+        unsigned const last = cap / NB16_GROUP - 1;
+        auto group_at = [&](unsigned g) { return lp[min(g, last) * WAVE]; };
+        float r[NS] = {};
+        if constexpr (STREAMS) {
+            // one lane per particle: both streams, one after the other (one set
+            // of sums in registers; both at once take 30 more, for a wave per
+            // SIMD less); two lanes: the lane's own
+            unsigned const end = mine ? n8 / NB16_GROUP : 0u;
+            unsigned s = part;
+            for (unsigned it = k - 1; it < 2u; ++it, ++s) {
+                stream a;
+                uint4 w0 = group_at(s), w1 = group_at(s + 2);
+                for (unsigned g = s; g < end; g += 4) {
+                    uint4 const n0 = group_at(g + 4), n1 = group_at(g + 6);
+                    group(a, w0);
+                    if (g + 2 < end) group(a, w1);
+                    fold(a);
+                    w0 = n0;
+                    w1 = n1;
                 }
+#pragma unroll
+                for (int c = 0; c < NS; ++c) r[c] += a.f[c] - a.c[c];
             }
-            rx = sx - ex;
-            ry = sy - ey;
-            rz = sz - ez;
-            if (AUX) {
-                en = acc[0]; s0 = acc[1]; s1 = acc[2]; s2 = acc[3]; s3 = acc[4]; s4 = acc[5]; s5 = acc[6];
+            if (k > 1) {   // wave-uniform
+                int const sl = int(lane + active < WAVE ? lane + active : lane);
+#pragma unroll
+                for (int c = 0; c < NS; ++c) r[c] += __shfl(r[c], sl, WAVE);
+            }
+        } else {
+            unsigned const nblk = (n8 / NB16_GROUP + 1) / 2;   // blocks of two groups
+            unsigned const b_begin = mine ? nblk * part / k : 0u;
+            unsigned const b_end = mine ? nblk * (part + 1) / k : 0u;
+            stream a;
+            uint4 w0 = group_at(2 * b_begin), w1 = group_at(2 * b_begin + 1);
+            for (unsigned b = b_begin; b < b_end; ++b) {
+                uint4 const n0 = group_at(2 * b + 2), n1 = group_at(2 * b + 3);
+                group(a, w0);
+                if (n8 - b * (2 * NB16_GROUP) > NB16_GROUP) group(a, w1);
+                fold(a);
+                w0 = n0;
+                w1 = n1;
+            }
+#pragma unroll
+            for (int c = 0; c < NS; ++c) r[c] = a.f[c] - a.c[c];
+            if (k > 1) {   // wave-uniform
+                // lane p (part 0) collects the runs of lanes p + active, ... in order
+                // (the shuffles read every lane's own run, never a running sum)
+                float sum[NS], comp[NS] = {};
+#pragma unroll
+                for (int c = 0; c < NS; ++c) sum[c] = r[c];
+                for (unsigned m = 1; m < k; ++m) {
+                    unsigned const src = lane + m * active;
+                    int const sl = int(src < WAVE ? src : lane);
+#pragma unroll
+                    for (int c = 0; c < NS; ++c) kahan_add(sum[c], comp[c], __shfl(r[c], sl, WAVE));
+                }
+#pragma unroll
+                for (int c = 0; c < NS; ++c) r[c] = sum[c] - comp[c];
             }
         }
         if (part != 0) continue;
+        float const rx = r[0], ry = r[1], rz = r[2];
+        float const en = AUX ? r[3 % NS] : 0.0f;
+        float sv[6] = {};
+        if constexpr (AUX)
+            for (int k = 0; k < 6; ++k) sv[k] = r[4 + k];
         float4 f;
         float sc[6];
         if (ISO) {
@@ -558,13 +584,12 @@ __device__ __forceinline__ float staged_force_segment(
             f = make_float4(separation_scale(rx, f_hi, f_lo), separation_scale(ry, f_hi, f_lo),
                             separation_scale(rz, f_hi, f_lo), AUX ? aux_weight * en : 0.0f);
             float const s2q = aux_weight * s_hi, s2l = aux_weight * s_lo;
-            float const sv[6] = {s0, s1, s2, s3, s4, s5};
 #pragma unroll
             for (int c = 0; c < 6; ++c) sc[c] = __builtin_fmaf(sv[c], s2q, sv[c] * s2l);
         } else {
             f = make_float4(rx, ry, rz, AUX ? aux_weight * en : 0.0f);
-            sc[0] = aux_weight * s0; sc[1] = aux_weight * s1; sc[2] = aux_weight * s2;
-            sc[3] = aux_weight * s3; sc[4] = aux_weight * s4; sc[5] = aux_weight * s5;
+#pragma unroll
+            for (int c = 0; c < 6; ++c) sc[c] = aux_weight * sv[c];
         }
         if (FUSE) {
             d2max = fmaxf(d2max, integrate_particle_f(F->pos, F->vel, f, F->image, F->posq_out, i, F->ip,
@@ -596,7 +621,7 @@ __device__ __forceinline__ float staged_force_segment(
 // again).  Each wave reads the 64 words itself, so the decision is uniform
 // without a barrier; workgroup 0 publishes the maximum to the host (chk.publish).
 
-template <int KIND, int TRUNC, bool AUX, bool ISO, bool MULTI, bool FUSE>
+template <int KIND, int TRUNC, bool AUX, bool ISO, bool MULTI, bool FUSE, bool STREAMS>
 __global__ __launch_bounds__(SEG_THREADS_MAX) void pair_force_staged_kernel(
     uint4 const* __restrict__ posq, uint32_t const* __restrict__ off, seg_params sp,
     uint16_t const* __restrict__ list, uint32_t const* __restrict__ count, unsigned cap, force_params P,
@@ -609,8 +634,9 @@ __global__ __launch_bounds__(SEG_THREADS_MAX) void pair_force_staged_kernel(
 
     unsigned const seg = seg_of_block(sp, blockIdx.x);   // workgroup 0 has segment 0
     if (seg >= sp.nseg) return;   // the whole workgroup
-    if (displacement_aborts(chk.slots, chk.bits, chk.publish, chk.seq)) return;   // the whole workgroup
-    float const d2 = staged_force_segment<KIND, TRUNC, AUX, ISO, MULTI, FUSE>(
+    // the whole workgroup
+    if (displacement_aborts(displacement_word(chk.slots), chk.slots, chk.bits, chk.publish, chk.seq)) return;
+    float const d2 = staged_force_segment<KIND, TRUNC, AUX, ISO, MULTI, FUSE, STREAMS>(
         posq, off, sp, seg, list, count, cap, P, force_zero, aux_weight, force, stress, stride, s_rec, st, s_pair, &F);
     if (FUSE) {
         wave_max_to(d2, disp_slot(F.disp_write));
@@ -668,9 +694,12 @@ __global__ __launch_bounds__(SEG_THREADS_MAX) void ens_force_kernel(
         F.ip = d.ip;
         F.pre_half_dt = E.pending ? d.ip.half_dt : 0.0f;
     }
-    float const d2 = staged_force_segment<KIND, TRUNC, AUX, true, MULTI, FUSE>(
-        posq + d.base, offsets + d.cell_base, d.sp, seg, list + d.list_off, count + d.base, d.cap, d.P, true, 0.5f,
-        force + d.base, AUX ? stress + d.base : nullptr, stride, s_rec, st, s_pair, &F);
+    auto const run = [&](auto streams) {
+        return staged_force_segment<KIND, TRUNC, AUX, true, MULTI, FUSE, decltype(streams)::value>(
+            posq + d.base, offsets + d.cell_base, d.sp, seg, list + d.list_off, count + d.base, d.cap, d.P, true, 0.5f,
+            force + d.base, AUX ? stress + d.base : nullptr, stride, s_rec, st, s_pair, &F);
+    };
+    float const d2 = force_streams(d.n) ? run(std::true_type{}) : run(std::false_type{});   // workgroup-uniform
     if (FUSE) wave_max_to(d2, ens_disp_slot(E, sys));
 }
 
@@ -826,6 +855,7 @@ void dispatch_trunc(force_launch const& a) {
 
 struct staged_launch {
     uint4 const* posq;
+    unsigned n;
     uint32_t const* off;
     seg_params const& sp;
     uint16_t const* list;
@@ -842,21 +872,26 @@ struct staged_launch {
     hipStream_t s;
 };
 
-template <int KIND, int TRUNC, bool AUX, bool ISO, bool MULTI>
+template <int KIND, int TRUNC, bool AUX, bool ISO, bool MULTI, bool STREAMS>
 void staged_go(staged_launch const& a) {
     size_t const lds = size_t(a.sp.lds_cap) * sizeof(uint4);
     unsigned const grid = SEG_XCD * a.sp.chunk;
     if constexpr (!AUX) {
         if (a.fuse) {
-            pair_force_staged_kernel<KIND, TRUNC, false, ISO, MULTI, true><<<grid, a.sp.threads, lds, a.s>>>(
+            pair_force_staged_kernel<KIND, TRUNC, false, ISO, MULTI, true, STREAMS><<<grid, a.sp.threads, lds, a.s>>>(
                 a.posq, a.off, a.sp, a.list, a.count, a.cap, a.p, true, a.w, a.force, a.stress, a.stride,
                 a.chk, *a.fuse);
             return;
         }
     }
-    pair_force_staged_kernel<KIND, TRUNC, AUX, ISO, MULTI, false><<<grid, a.sp.threads, lds, a.s>>>(
+    pair_force_staged_kernel<KIND, TRUNC, AUX, ISO, MULTI, false, STREAMS><<<grid, a.sp.threads, lds, a.s>>>(
         a.posq, a.off, a.sp, a.list, a.count, a.cap, a.p, a.force_zero, a.w, a.force, a.stress, a.stride,
         a.chk, fused_integrate{});
+}
+template <int KIND, int TRUNC, bool AUX, bool ISO, bool MULTI>
+void staged_go(staged_launch const& a) {
+    force_streams(a.n) ? staged_go<KIND, TRUNC, AUX, ISO, MULTI, true>(a)
+                       : staged_go<KIND, TRUNC, AUX, ISO, MULTI, false>(a);
 }
 
 template <int KIND, int TRUNC>
@@ -1112,14 +1147,14 @@ void launch_pair_full(uint4 const* posq1, unsigned n1, uint4 const* posq2, unsig
     HIP_CHECK(hipGetLastError());
 }
 
-void launch_pair_force_staged(uint4 const* posq, uint32_t const* offset, seg_params const& sp, uint16_t const* list,
-                              uint32_t const* count, unsigned cap, force_params const& p, bool aux, bool force_zero,
+void launch_pair_force_staged(uint4 const* posq, unsigned n, uint32_t const* offset, seg_params const& sp,
+                              uint16_t const* list, uint32_t const* count, unsigned cap, force_params const& p, bool aux, bool force_zero,
                               float aux_weight, float4* force, float* stress, unsigned stride, hipStream_t s,
                               displacement_check const* check, fused_integrate const* fuse) {
     if (!sp.nseg) return;
     if (fuse && aux) throw error(HALMD_ERR_INVALID_ARGUMENT, "pair force: the fused step has no aux path");
     displacement_check const chk = check ? *check : displacement_check{};
-    staged_launch const a{posq,  offset, sp,     list,   count, cap, p,    aux, force_zero, aux_weight,
+    staged_launch const a{posq,  n,      offset, sp,     list,   count, cap, p,    aux, force_zero, aux_weight,
                           force, stress, stride, chk,    fuse,  s};
     if (p.kind == POTENTIAL_LENNARD_JONES)
         staged_trunc<POTENTIAL_LENNARD_JONES>(a);

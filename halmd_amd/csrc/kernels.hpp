@@ -42,11 +42,13 @@ void launch_fill_u32(uint32_t* out, uint32_t value, size_t n, hipStream_t s);
 void launch_copy(void const* src, void* dst, size_t bytes, hipStream_t s);
 // n words (a kernel rather than a DMA copy: shorter latency for small arrays)
 void launch_copy_u32(uint32_t const* src, uint32_t* dst, size_t n, hipStream_t s);
-// dst[k] := (seq << 32) | *src.word[k] for k < n (MAILBOX_WORDS at most; a
-// null source reads as 0), stored at system scope into host-mapped memory
+// dst[k] := (seq << 32) | the largest of the count[k] (at most 64) words
+// stride[k] apart at word[k], for k < n (MAILBOX_WORDS at most; a null source
+// reads as 0), stored at system scope into host-mapped memory
 constexpr unsigned MAILBOX_WORDS = 4;
 struct mailbox_sources {
     uint32_t const* word[MAILBOX_WORDS];
+    unsigned count[MAILBOX_WORDS], stride[MAILBOX_WORDS];
 };
 void launch_post_words(mailbox_sources const& src, unsigned n, unsigned long long* dst, uint32_t seq, hipStream_t s);
 // VALU rate probe (blocks workgroups of 256 threads); returns the number of
@@ -220,27 +222,36 @@ __host__ __device__ inline void seg_own_row(seg_params const& sp, seg_place cons
 // 16-bit slot lists (an entry is the byte offset 16 * slot of the record in
 // the staged union, so a union holds at most 4096 records): entry k of
 // particle i (memory order) at
-// (i / 64) * 64 * cap + (k / 16) * 1024 + (i % 64) * 16 + k % 16 (uint16 units;
-// one lane block = 16 entries = 32 bytes, the write granule of the memory
-// system; cap a multiple of 16)
-constexpr unsigned NB16_BLOCK = 16;
+// (i / 64) * 64 * cap + (k / 8) * 512 + (i % 64) * 8 + k % 8 (uint16 units; a
+// group of 8 entries is one load of a lane, and a wave's 64 groups are 1 KiB in
+// a row)
+constexpr unsigned NB16_GROUP = 8;
+constexpr unsigned NB16_BLOCK = 16;   // (list capacities are multiples of it)
 constexpr unsigned SEG_MAX_RECORDS = 4096;   // staged union plus sentinel
 __host__ __device__ inline size_t list16_index(size_t i, size_t k, size_t cap) {
-    return (i & ~size_t(WAVE - 1)) * cap + (k / NB16_BLOCK) * WAVE * NB16_BLOCK + (i & (WAVE - 1)) * NB16_BLOCK +
-           k % NB16_BLOCK;
+    return (i & ~size_t(WAVE - 1)) * cap + (k / NB16_GROUP) * WAVE * NB16_GROUP + (i & (WAVE - 1)) * NB16_GROUP +
+           k % NB16_GROUP;
 }
+constexpr unsigned STAT_SLOTS = 64, STAT_STRIDE = 32;   // (128 bytes apart)
+// Single systems below BUILD_SPLIT_BELOW particles build their lists by three
+// waves per 64 particles: 27 against 48 us at N = 4000, 43 against 64 us at
+// N = 64,000, 63 us either way at N = 108,000, 210 against 146 us at N = 524,288.
+constexpr unsigned BUILD_SPLIT_BELOW = 1u << 17;
 // Lists are padded with the slot U of a sentinel record (staged after the
 // union, at least a third of the box away from every particle of the segment
 // in y and z) to a multiple of 8 entries; count[i] excludes the padding.
-// stats[0]: largest count (may exceed cap); stats[1]: largest staging size
-// U + 1 (a segment whose staging exceeds sp.lds_cap builds nothing; the caller
-// retries)
+// stats: STAT_SLOTS pairs of words STAT_STRIDE apart, whose largest values are
+// the largest count (may exceed cap) and the largest staging size U + 1 (a
+// segment whose staging exceeds sp.lds_cap builds nothing; the caller retries).
+// Workgroup b raises pair b % STAT_SLOTS: atomics on one word take about 15 ns
+// each on this chip whatever else it does, and the 23,000 of a build at N =
+// 2^20 on one word took all of its 370 us.
 //
 // With sub_offset (the offsets of the (cell, x sub-bin) order the particles
 // are in, ncells SUB_BINS + 1 entries; cubic box, nx >= 4) each lane scans
 // only the candidate windows its position allows (same lists); the dynamic
 // LDS is then windowed_build_lds() bytes.
-void launch_build_neighbours_staged(uint4 const* posq, uint32_t const* offset, seg_params const& sp,
+void launch_build_neighbours_staged(uint4 const* posq, unsigned n, uint32_t const* offset, seg_params const& sp,
                                     neighbour_params const& p, unsigned cap, uint16_t* list, uint32_t* count,
                                     uint32_t* stats, hipStream_t s, uint32_t const* sub_offset = nullptr);
 constexpr unsigned WIN_MAX = 10;   // candidate windows per lane: 9 rows, the own row split
@@ -338,12 +349,19 @@ struct displacement_check {
 };
 constexpr unsigned PUBLISH_RING = 4;
 
+// Systems below FORCE_STREAMS_BELOW particles sum each particle's force in two
+// streams (force.hip), a result that does not depend on the segment shape;
+// larger ones in one pass: equal at N = 256,000 (35 us), 53 against 51 us at
+// N = 524,288, 102 against 93 us at N = 2^20.
+constexpr unsigned FORCE_STREAMS_BELOW = 1u << 18;
+__host__ __device__ inline bool force_streams(unsigned n) { return n < FORCE_STREAMS_BELOW; }
 // the same over 16-bit slot lists of cell segments (particles in cell order);
 // check (optional): a speculative launch; fuse (optional, no aux): integrate
 // each particle instead of writing its force
-void launch_pair_force_staged(uint4 const* posq, uint32_t const* offset, seg_params const& sp, uint16_t const* list,
-                              uint32_t const* count, unsigned cap, force_params const& p, bool aux, bool force_zero,
-                              float aux_weight, float4* force, float* stress, unsigned stride, hipStream_t s,
+void launch_pair_force_staged(uint4 const* posq, unsigned n, uint32_t const* offset, seg_params const& sp,
+                              uint16_t const* list, uint32_t const* count, unsigned cap, force_params const& p,
+                              bool aux, bool force_zero, float aux_weight, float4* force, float* stress,
+                              unsigned stride, hipStream_t s,
                               displacement_check const* check = nullptr, fused_integrate const* fuse = nullptr);
 
 // ---------------------------------------------------------------------------

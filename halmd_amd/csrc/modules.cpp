@@ -1032,7 +1032,7 @@ void neighbour::init(double const* rc, unsigned nt1, unsigned nt2) {
     double const rho = double(p2.n) / b.volume();
     double const nmean = 4.0 / 3.0 * M_PI * std::pow(rc_max + r_skin, 3) * rho;
     count.resize(p.n);
-    d_maxcount.resize(2);
+    d_maxcount.resize(STAT_SLOTS * STAT_STRIDE);
     h_maxcount.resize(2);
     // the first neighbour module of a particle instance keeps it in cell order
     // and uses the cell-segment kernels; the rules need nx >= 3 (S <= nx - 2)
@@ -1055,13 +1055,9 @@ void neighbour::init(double const* rc, unsigned nt1, unsigned nt2) {
         // at N = 2^20, with a third sort pass in the binning)
         char const* ew = std::getenv("HALMD_LIST_WINDOWS");
         windows = params.iso && bin->grid.ncell[0] >= 4 && ew && std::atoi(ew) != 0;
-        // about `target` particles per segment (per 256-thread workgroup) at
-        // the mean cell occupancy (pair_trunc::tune refines the width by
-        // measurement); HALMD_SEG_TARGET overrides the target
-        double target = 200;
-        if (char const* e = std::getenv("HALMD_SEG_TARGET")) target = std::max(1.0, std::atof(e));
+        // (pair_trunc::tune refines the width by measurement)
         unsigned S, R;
-        segment_shape(mean_occupancy(), bin->grid, target, S, R);
+        segment_shape(mean_occupancy(), bin->grid, segment_target(p.n), S, R);
         set_segments(S, R, SEG_THREADS_MAX);
     } else {
         cap = unsigned(round_up(size_t(std::ceil(nmean / occupancy)) + NB_BLOCK, NB_BLOCK));
@@ -1106,6 +1102,11 @@ void segment_shape(double occupancy, cell_grid const& g, double target, unsigned
     R = std::max(1u, std::min({R, SEG_RMAX, g.ncell[1] - 2}));
     S = unsigned(std::max(1.0, std::round(cells / R)));
     S = std::max(1u, std::min({S, SEG_MAX, g.ncell[0] - 2}));
+}
+
+double segment_target(unsigned) {
+    if (char const* e = std::getenv("HALMD_SEG_TARGET")) return std::max(1.0, std::atof(e));
+    return 200;   // about a workgroup's threads
 }
 
 double neighbour::mean_occupancy() const { return bin ? double(p.n) / bin->ncells : 0.0; }
@@ -1210,15 +1211,17 @@ void neighbour::update(double displacement_bound) {
     // then the segment lists
     bin->reorder_particles(windows, displacement_bound, disp.r0);
     while (true) {
-        launch_fill_u32(d_maxcount, 0u, 2, s);
+        launch_fill_u32(d_maxcount, 0u, d_maxcount.size(), s);
         timer.start(s);
         bool const win = windows && windowed_build_lds(sp) <= lds_bytes;
-        launch_build_neighbours_staged(p.posq, bin->order_offset, sp, params, cap, list16, count, d_maxcount, s,
+        launch_build_neighbours_staged(p.posq, p.n, bin->order_offset, sp, params, cap, list16, count, d_maxcount, s,
                                        win ? bin->order_sub_offset.get() : nullptr);
         timer.stop(s);
         // the largest count, the largest union and the merge check of the
         // binning (0 when it sorted), polled as they are stored
-        mailbox_sources const src{{d_maxcount.get(), d_maxcount.get() + 1, bin->merge_check_word(), nullptr}};
+        mailbox_sources const src{{d_maxcount.get(), d_maxcount.get() + 1, bin->merge_check_word(), nullptr},
+                                  {STAT_SLOTS, STAT_SLOTS, 1, 0},
+                                  {STAT_STRIDE, STAT_STRIDE, 1, 0}};
         uint32_t got[3];
         build_box.wait(build_box.post(src, 3, s), 3, got, s);
         bin->merge_checked(got[2]);
@@ -1471,7 +1474,7 @@ bool pair_trunc::launch(bool force_zero, displacement_check const* check, fused_
     }
     timer.start(p.stream);
     if (nb.staged)
-        launch_pair_force_staged(p.posq, nb.bin->order_offset, nb.sp_force, nb.list16, nb.count, nb.cap, params, aux,
+        launch_pair_force_staged(p.posq, p.n, nb.bin->order_offset, nb.sp_force, nb.list16, nb.count, nb.cap, params, aux,
                                  force_zero, w, p.force, p.stress, p.n_pad, p.stream, check, fuse);
     else
         launch_pair_force(p.posq, p.n, nb.list, nb.count, nb.cap, params, aux, force_zero, w, p.force, p.stress,

@@ -336,6 +336,10 @@ class hilbert;
 // particles at the given mean cell occupancy (within the grid's limits)
 void segment_shape(double occupancy, cell_grid const& g, double target, unsigned& S, unsigned& R);
 
+// particles per segment of a system of n particles that has the chip to itself
+// (HALMD_SEG_TARGET overrides)
+double segment_target(unsigned n);
+
 class neighbour {
 public:
     // bin == nullptr: lists from all particle pairs (from_particle), for

@@ -176,14 +176,16 @@ __global__ void copy_u32_kernel(uint32_t const* __restrict__ a, uint32_t* __rest
     if (i < n) a_out[i] = a[i];
 }
 
-// word k of a mailbox: (seq << 32) | *src.word[k] (0 for a null source), one
-// system-scope store into host-mapped memory
-__global__ void post_words_kernel(mailbox_sources src, unsigned n, unsigned long long* dst, uint32_t seq) {
-    unsigned const k = threadIdx.x;
-    if (k >= n) return;
-    uint32_t const v = src.word[k] ? *src.word[k] : 0u;
-    __hip_atomic_store(dst + k, (static_cast<unsigned long long>(seq) << 32) | v, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_SYSTEM);
+// word k of a mailbox, by wave k: (seq << 32) | the largest of the source's
+// words (0 for a null source), one system-scope store into host-mapped memory
+__global__ void post_words_kernel(mailbox_sources src, unsigned long long* dst, uint32_t seq) {
+    unsigned const k = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    uint32_t v = 0;
+    if (src.word[k] && lane < src.count[k]) v = src.word[k][lane * src.stride[k]];
+    v = wave_max_u32(v);
+    if (lane == 0)
+        __hip_atomic_store(dst + k, (static_cast<unsigned long long>(seq) << 32) | v, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ void iota_copy_kernel(uint32_t* __restrict__ out, size_t n, uint32_t const* __restrict__ src,
@@ -408,7 +410,8 @@ void launch_copy(void const* src, void* dst, size_t bytes, hipStream_t s) {
 void launch_post_words(mailbox_sources const& src, unsigned n, unsigned long long* dst, uint32_t seq,
                        hipStream_t s) {
     if (n > MAILBOX_WORDS) throw error(HALMD_ERR_INVALID_ARGUMENT, "mailbox: too many words");
-    post_words_kernel<<<1, WAVE, 0, s>>>(src, n, dst, seq);
+    if (!n) return;
+    post_words_kernel<<<1, n * WAVE, 0, s>>>(src, dst, seq);
     HIP_CHECK(hipGetLastError());
 }
 
