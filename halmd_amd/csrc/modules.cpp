@@ -1104,9 +1104,21 @@ void segment_shape(double occupancy, cell_grid const& g, double target, unsigned
     S = std::max(1u, std::min({S, SEG_MAX, g.ncell[0] - 2}));
 }
 
-double segment_target(unsigned) {
+double segment_target(unsigned n) {
     if (char const* e = std::getenv("HALMD_SEG_TARGET")) return std::max(1.0, std::atof(e));
-    return 200;   // about a workgroup's threads
+    // The staging of a segment's union is paid per segment, so up to the 256
+    // threads of a workgroup larger is better where there are workgroups enough;
+    // below N = 160,000 there are not, and about 800 segments are best: the
+    // whole step (force, integration, its share of the list build) takes 22
+    // against 28 us with segments of 200 at N = 4000, 20 against 28 at 16,000,
+    // 22 against 26 at 64,000, 35 against 39 at 108,000, the same from 160,000.
+    // (One to two cells a segment at the least: smaller workgroups stage more
+    // than they own.)
+    if (n < FORCE_STREAMS_BELOW) return std::clamp(n / 800.0, 32.0, 200.0);
+    // Here the sums follow the shape, so an ensemble's systems of this size
+    // take the same (200 against 230: 76 against 80 us at N = 524,288, 140
+    // against 136 at N = 2^20).
+    return n < 3 * FORCE_STREAMS_BELOW ? 200 : 230;
 }
 
 double neighbour::mean_occupancy() const { return bin ? double(p.n) / bin->ncells : 0.0; }
