@@ -44,10 +44,11 @@ void launch_copy(void const* src, void* dst, size_t bytes, hipStream_t s);
 void launch_copy_u32(uint32_t const* src, uint32_t* dst, size_t n, hipStream_t s);
 // dst[k] := (seq << 32) | the largest of the count[k] (at most 64) words
 // stride[k] apart at word[k], for k < n (MAILBOX_WORDS at most; a null source
-// reads as 0), stored at system scope into host-mapped memory
+// reads as 0), stored at system scope into host-mapped memory; the words read
+// are set to 0 (for their next writers, without a fill of their own)
 constexpr unsigned MAILBOX_WORDS = 4;
 struct mailbox_sources {
-    uint32_t const* word[MAILBOX_WORDS];
+    uint32_t* word[MAILBOX_WORDS];
     unsigned count[MAILBOX_WORDS], stride[MAILBOX_WORDS];
 };
 void launch_post_words(mailbox_sources const& src, unsigned n, unsigned long long* dst, uint32_t seq, hipStream_t s);
@@ -527,8 +528,8 @@ void launch_ens_decide(ens_desc const* descs, unsigned nsys, uint32_t const* ski
 // + e in ascending index, the particles that moved by -e, in memory order.
 //  - rank: waves over runs of old cells; keys[i] = new cell | code(e) << 27,
 //    vals[i] = rank of i among the particles of its old cell with that code,
-//    cnt27[27 c' + code] = their number
-//  - cell_count: one thread per new cell; base27[27 c + code] = particles
+//    cnt27[code n_cells + c'] = their number
+//  - cell_count: one thread per new cell; base27[code n_cells + c] = particles
 //    that reach c from sources below c + e, offsets_t = the exclusive scan of
 //    the counts within each block of ENS_CELL_BLOCK cells, bsum = block sums
 //  - cell_carry: the sums of the earlier blocks added (offsets_t final)
@@ -562,21 +563,38 @@ constexpr unsigned ENS_CELL_KEY_BITS = 27;   // cells per system below 2^27
 // The same merge for one particle instance: the stable cell order of its
 // present positions from the cell order of its previous binning (old_offsets
 // describe the memory order; every particle has moved at most into one of the
-// 26 cells around its old one).  Writes new_offsets (n_cells + 1 entries) and
-// perm (the gather list of the new order); flag receives ENS_SKIP_FAR if a
-// particle moved farther (then new_offsets and perm are not written).  The
-// tables come from merge_tables_upload for this grid and n.
+// 26 cells around its old one).  launch_merge_cell_order finds each particle's
+// slot (in the scratch); flag receives ENS_SKIP_FAR if a particle moved farther
+// (0 before).  launch_merge_scatter moves the particles there, and writes the
+// n_cells + 1 offsets to both arrays and the identity to vals; with flag set it
+// keeps every particle's slot and the offsets.  The tables come from
+// merge_tables_upload for this grid and n.
 struct merge_scratch {
     ens_desc* desc;         // 1 descriptor
     uint32_t* work;         // ens_work_words(1) words
     uint32_t *keys, *rank;  // n words each
-    uint32_t *cnt27, *base27, *bsum;   // 27 n_cells, 27 n_cells, n_cells / ENS_CELL_BLOCK + 2 words
-    uint32_t* flag;         // 1 word
-    unsigned n = 0, ncells = 0;   // set by merge_tables_upload
+    uint32_t *cnt27, *base27, *first, *bsum;   // 27 n_cells, 27 n_cells, n_cells, n_cells / ENS_CELL_BLOCK + 2 words
+    uint32_t *flag, *ticket;   // 1 word each, 0 before the first use
+    cell_grid grid;
+    unsigned n, ncells;
 };
-void merge_tables_upload(cell_grid const& g, unsigned n, merge_scratch& m, hipStream_t s);
-void launch_merge_cell_order(uint4 const* posq, uint32_t const* old_offsets, uint32_t* new_offsets, uint32_t* perm,
-                             merge_scratch const& m, hipStream_t s);
+// a particle instance's arrays and the ones that receive the new order
+struct rearrange_arrays {
+    float4 const *pos_in, *vel_in;
+    int4 const* image_in;
+    uint32_t const* id_in;
+    uint4 const* posq_in;
+    float4 *pos_out, *vel_out;
+    int4* image_out;
+    uint32_t* id_out;
+    uint4* posq_out;
+    uint32_t* rid;   // the reverse map
+    float4* r0;      // optional: the new order's positions (hi words)
+};
+void merge_tables_upload(cell_grid const& g, unsigned n, merge_scratch const& m, hipStream_t s);
+void launch_merge_cell_order(uint4 const* posq, uint32_t const* old_offsets, merge_scratch const& m, hipStream_t s);
+void launch_merge_scatter(rearrange_arrays const& a, merge_scratch const& m, uint32_t* offsets,
+                          uint32_t* order_offsets, uint32_t* vals, hipStream_t s);
 // per-system FP64 sums, one workgroup per listed system: out[4 s] = sum m v^2
 // (velocities after the pending kick, when pending), [1] = sum en_pot, [2] =
 // sum of the stress traces (both from aux_force / stress when given), [3] = n

@@ -419,6 +419,15 @@ void particle::evaluate_forces() {
     }
 }
 
+void particle::rearrange_merged(merge_scratch const& m, uint32_t* offsets, uint32_t* order_offsets, uint32_t* vals,
+                                float4* r0) {
+    if (force_valid) settle_velocity();   // as below
+    rearrange_arrays const a{pos,     vel,     image,     id,     posq,     pos_alt,    vel_alt,
+                             image_alt, id_alt, posq_alt, reverse_id, r0};
+    launch_merge_scatter(a, m, offsets, order_offsets, vals, stream);
+    adopt_rearranged();
+}
+
 void particle::rearrange(uint32_t const* perm, float4* r0) {
     // a kick owed with a force not yet evaluated stays owed (the force will be
     // evaluated in the new order); one whose force is in memory is applied,
@@ -426,6 +435,10 @@ void particle::rearrange(uint32_t const* perm, float4* r0) {
     if (force_valid) settle_velocity();
     launch_rearrange(pos, vel, image, id, posq, perm, n, pos_alt, vel_alt, image_alt, id_alt, posq_alt, stream,
                      reverse_id, r0);
+    adopt_rearranged();
+}
+
+void particle::adopt_rearranged() {
     std::swap(posq, posq_alt);
     std::swap(pos, pos_alt);
     std::swap(vel, vel_alt);
@@ -727,6 +740,7 @@ void binning::reorder_particles(bool sub_bins, double displacement_bound, float4
     if (merge_flag_pending) {
         // the last merge's check, when no list build read it
         HIP_CHECK(hipMemcpyAsync(h_merge_flag.get(), merge_flag.get(), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        launch_fill_u32(merge_flag, 0u, 1, s);
         p.sync();
         merge_checked(h_merge_flag[0]);
     }
@@ -744,19 +758,17 @@ void binning::reorder_particles(bool sub_bins, double displacement_bound, float4
             merge_cnt27.resize(27 * size_t(ncells));
             merge_base27.resize(27 * size_t(ncells));
             merge_bsum.resize(ncells / ENS_CELL_BLOCK + 2);
-            merge_flag.resize(1);
+            merge_first.resize(ncells);
+            merge_flag.resize(2);   // the flag and the ticket
+            launch_fill_u32(merge_flag, 0u, 2, s);
             h_merge_flag.resize(1);
-            merge_scratch m{merge_desc, merge_work, keys, merge_rank, merge_cnt27, merge_base27, merge_bsum,
-                            merge_flag};
-            merge_tables_upload(grid, p.n, m, s);
+            merge_tables_upload(grid, p.n, merge_buffers(), s);
         }
-        merge_scratch m{merge_desc, merge_work, keys, merge_rank, merge_cnt27, merge_base27, merge_bsum, merge_flag};
-        m.n = p.n;
-        m.ncells = ncells;
+        merge_scratch const m = merge_buffers();
         timer.start(s);
-        launch_merge_cell_order(p.posq, order_offset, offset, vals, m, s);
-        merge_flag_pending = true;   // read by the list build that follows (merge_check_word)
-        p.rearrange(vals, r0);
+        launch_merge_cell_order(p.posq, order_offset, m, s);
+        merge_flag_pending = true;   // read and reset after the list build that follows (merge_check_word)
+        p.rearrange_merged(m, offset, order_offset, vals, r0);
         ++merges;
     } else if (!sub_bins) {
         update(false);
@@ -778,7 +790,7 @@ void binning::reorder_particles(bool sub_bins, double displacement_bound, float4
         launch_cell_offsets(keys, p.n, ncells << SUB_BITS, order_sub_offset, s, 0);
     }
     // sorted order is now memory order; the offsets describe it
-    launch_iota_copy_u32(vals, p.n, offset.get(), order_offset.get(), order_offset.size(), s);
+    if (!merge) launch_iota_copy_u32(vals, p.n, offset.get(), order_offset.get(), order_offset.size(), s);
     timer.stop(s);
     // offsets describe the new order as well (the keys only after a sort)
     version = p.position_version;
@@ -786,7 +798,12 @@ void binning::reorder_particles(bool sub_bins, double displacement_bound, float4
     reordered_version = p.order_version;
 }
 
-uint32_t const* binning::merge_check_word() const { return merge_flag_pending ? merge_flag.get() : nullptr; }
+uint32_t* binning::merge_check_word() { return merge_flag_pending ? merge_flag.get() : nullptr; }
+
+merge_scratch binning::merge_buffers() {
+    return {merge_desc, merge_work, keys, merge_rank, merge_cnt27, merge_base27, merge_first, merge_bsum,
+            merge_flag.get(), merge_flag.get() + 1, grid, p.n, ncells};
+}
 
 void binning::merge_checked(uint32_t flag) {
     if (!merge_flag_pending) return;
@@ -1033,6 +1050,7 @@ void neighbour::init(double const* rc, unsigned nt1, unsigned nt2) {
     double const nmean = 4.0 / 3.0 * M_PI * std::pow(rc_max + r_skin, 3) * rho;
     count.resize(p.n);
     d_maxcount.resize(STAT_SLOTS * STAT_STRIDE);
+    launch_fill_u32(d_maxcount, 0u, d_maxcount.size(), p.stream);   // (reset as they are read)
     h_maxcount.resize(2);
     // the first neighbour module of a particle instance keeps it in cell order
     // and uses the cell-segment kernels; the rules need nx >= 3 (S <= nx - 2)
@@ -1223,14 +1241,13 @@ void neighbour::update(double displacement_bound) {
     // then the segment lists
     bin->reorder_particles(windows, displacement_bound, disp.r0);
     while (true) {
-        launch_fill_u32(d_maxcount, 0u, d_maxcount.size(), s);
         timer.start(s);
         bool const win = windows && windowed_build_lds(sp) <= lds_bytes;
         launch_build_neighbours_staged(p.posq, p.n, bin->order_offset, sp, params, cap, list16, count, d_maxcount, s,
                                        win ? bin->order_sub_offset.get() : nullptr);
         timer.stop(s);
         // the largest count, the largest union and the merge check of the
-        // binning (0 when it sorted), polled as they are stored
+        // binning (0 when it sorted), polled as they are stored, and reset
         mailbox_sources const src{{d_maxcount.get(), d_maxcount.get() + 1, bin->merge_check_word(), nullptr},
                                   {STAT_SLOTS, STAT_SLOTS, 1, 0},
                                   {STAT_STRIDE, STAT_STRIDE, 1, 0}};

@@ -169,9 +169,13 @@ public:
     // r0 (optional): also receives the new order's positions (hi words), the
     // reference positions of a displacement tracker reset at the same point
     void rearrange(uint32_t const* perm, float4* r0 = nullptr);
+    // the same into the order of a merge (launch_merge_scatter)
+    void rearrange_merged(merge_scratch const& m, uint32_t* offsets, uint32_t* order_offsets, uint32_t* vals,
+                          float4* r0);
     void sync();
 
 private:
+    void adopt_rearranged();   // the other arrays take over
     void download_hilo(dbuf<float4> const& b, double* out);
     void upload_hilo(dbuf<float4>& b, double const* in, bool species);
     std::vector<float4> host_tmp_;
@@ -246,13 +250,14 @@ public:
     bool sub_order = false;            // the last reorder used sub-bins
     uint64_t reordered_version = ~uint64_t(0);   // particle order version this binning's last reorder left
     dbuf<ens_desc> merge_desc;
-    dbuf<uint32_t> merge_work, merge_rank, merge_cnt27, merge_base27, merge_bsum, merge_flag;
+    dbuf<uint32_t> merge_work, merge_rank, merge_cnt27, merge_base27, merge_first, merge_bsum, merge_flag;
+    merge_scratch merge_buffers();
     hbuf<uint32_t> h_merge_flag;
     bool merge_flag_pending = false;   // the last merge's flag is still to be checked
     // the device word of the pending merge check (null: none pending); the
     // caller that reads it after the merge hands its value to merge_checked,
     // which throws when a particle left the 27 cells around its old one
-    uint32_t const* merge_check_word() const;
+    uint32_t* merge_check_word();
     void merge_checked(uint32_t flag);
     void cell_lists(unsigned* begin_out, unsigned* end_out, unsigned* index_out);
     kernel_timer timer;

@@ -181,7 +181,10 @@ __global__ void copy_u32_kernel(uint32_t const* __restrict__ a, uint32_t* __rest
 __global__ void post_words_kernel(mailbox_sources src, unsigned long long* dst, uint32_t seq) {
     unsigned const k = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     uint32_t v = 0;
-    if (src.word[k] && lane < src.count[k]) v = src.word[k][lane * src.stride[k]];
+    if (src.word[k] && lane < src.count[k]) {
+        v = src.word[k][lane * src.stride[k]];
+        src.word[k][lane * src.stride[k]] = 0;
+    }
     v = wave_max_u32(v);
     if (lane == 0)
         __hip_atomic_store(dst + k, (static_cast<unsigned long long>(seq) << 32) | v, __ATOMIC_RELAXED,

@@ -3,8 +3,8 @@
 Between two rebuilds the displacement check bounds every particle's move by
 about half the skin, far less than a cell, so the particles reach at most the
 26 cells around their old one and the new stable cell order is a merge of the
-old one (binning.hip: ens_rank_kernel, ens_cell_count_kernel,
-ens_cell_carry_kernel, ens_order_kernel).  A rebuild after another
+old one (binning.hip: ens_rank_kernel, merge_count_kernel,
+merge_scatter_kernel).  A rebuild after another
 rearrangement (here the Hilbert sort every 100 steps) sorts.
 """
 import numpy as np
@@ -61,3 +61,20 @@ def test_merged_cell_order_is_the_sorted_one(monkeypatch, box):
     print("rebuilds", a.neighbour.rebuilds, "merged", merged, "sorted", sorted_)
     assert merged > 0 and sorted_ >= 1
     assert b.neighbour.reorders[0] == 0
+
+
+def test_merge_over_many_blocks_of_cells(monkeypatch):
+    # 44 cells a side: more blocks of 256 cells (333) than the workgroup that
+    # adds them up has threads
+    runs = []
+    for merge in ("1", "0"):
+        monkeypatch.setenv("HALMD_BINNING_MERGE", merge)
+        w = workloads.lennard_jones(20000, density=0.025, r_cut=1.8, temperature=1.2, seed=9, timestep=0.005,
+                                    sort_interval=100)
+        assert np.prod(w.neighbour.binning.ncell) > 256 * 256
+        w.sampler.run(150)
+        runs.append(w)
+    a, b = runs
+    for name in ("position", "velocity", "image"):
+        assert np.array_equal(a.particle.ordered(name), b.particle.ordered(name)), name
+    assert a.neighbour.reorders[0] > 0 and b.neighbour.reorders[0] == 0
