@@ -47,12 +47,18 @@ __device__ __forceinline__ ff ff_from_double(double x) {
 // fixed-point snapshot (into posq) of particle i; returns |r - r0|^2 (0
 // without r0).  Shared by the single-system and ensemble integrate kernels and
 // the pair-force kernel that integrates its particles as it finishes them.
+// (thermostat: called with the velocity, mass and force after the deferred kick)
+struct no_thermostat {
+    __device__ void operator()(ff&, ff&, ff&, float, float4) const {}
+};
+template <typename Thermostat = no_thermostat>
 __device__ __forceinline__ float integrate_particle_f(float4* __restrict__ pos, float4* __restrict__ vel,
                                                      float4 const f, int4* __restrict__ image,
                                                      uint4* __restrict__ posq, unsigned i,
                                                      integrate_params const& p, float pre_half_dt,
                                                      double const* __restrict__ scale,
-                                                     float4 const* __restrict__ r0) {
+                                                     float4 const* __restrict__ r0,
+                                                     Thermostat const& thermostat = Thermostat()) {
     float d2 = 0.0f;
     // every load up front (r0 too): a load issued after the stores would
     // wait for them and add a second memory round trip to each wave
@@ -68,6 +74,7 @@ __device__ __forceinline__ float integrate_particle_f(float4* __restrict__ pos, 
         vy = ff_add_f(vy, f.y * k);
         vz = ff_add_f(vz, f.z * k);
     }
+    thermostat(vx, vy, vz, m, f);
     if (scale) {
         ff const s = ff_from_double(*scale);
         vx = ff_mul(vx, s); vy = ff_mul(vy, s); vz = ff_mul(vz, s);

@@ -381,18 +381,25 @@ constexpr unsigned DISP_SET = DISP_SLOTS * DISP_STRIDE;   // words per slot set
 // device) and optional max-displacement tracking against r0 (max |r - r0|^2 as
 // float bits folded into the slot set at max_disp2; the slots of the set at
 // clear_slot, that of the next step, are set to zero)
+// (bath: the Andersen finalize of the previous step first, with no pre_half_dt
+// and no scale)
+struct andersen_step {
+    uint32_t const* id;
+    float half_dt, coll_prob, sqrt_temperature;
+    uint64_t seed, step;   // the counter of its random numbers, with the particle's id
+};
 void launch_verlet_integrate(float4* pos, float4* vel, float4 const* force, int4* image, uint4* posq, unsigned n,
                              integrate_params const& p, float pre_half_dt, double const* scale, float4 const* r0,
-                             uint32_t* max_disp2, uint32_t* clear_slot, hipStream_t s);
+                             uint32_t* max_disp2, uint32_t* clear_slot, hipStream_t s,
+                             andersen_step const* bath = nullptr);
 void launch_verlet_finalize(float4* vel, float4 const* force, unsigned n, float half_dt, hipStream_t s);
 void launch_rescale_velocity(float4* vel, unsigned n, double const* scale, hipStream_t s);
 void launch_copy_hi(float4 const* pos, float4* r0, unsigned n, hipStream_t s);
 void launch_max_displacement(float4 const* pos, float4 const* r0, unsigned n, float const* L, float const* invL,
                              uint32_t* max_disp2, hipStream_t s);
-// Andersen collisions: with probability p per particle resample v ~ N(0, sqrt(T))
-// (counter-based RNG keyed by seed, step and particle id), else kick
-void launch_andersen_finalize(float4* vel, float4 const* force, uint32_t const* id, unsigned n, float half_dt,
-                              float coll_prob, float sqrt_temperature, uint64_t seed, uint64_t step, hipStream_t s);
+// the Andersen finalize: the kick, or with probability coll_prob per particle a
+// resampled velocity v ~ N(0, sqrt(T))
+void launch_andersen_finalize(float4* vel, float4 const* force, unsigned n, andersen_step const& t, hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // ensembles: many independent systems in shared arrays (ensemble.cpp drives
@@ -622,9 +629,14 @@ struct nhc_state {
     double scale;           // last velocity scale factor
     double en_nhc_raw;      // T (dN xi0 + xi1) + sum m_xi v_xi^2 / 2 (not divided by N)
 };
-// sum m v^2 partials -> chain half-step; writes state->scale
-void launch_nhc_propagate(double const* partials, nhc_state* state, hipStream_t s);
+// sum m v^2 partials -> chain half-step; writes state->scale.  two: a second
+// half-step follows, from the sum that the first one's scale leaves; scale is
+// their product
+void launch_nhc_propagate(double const* partials, nhc_state* state, bool two, hipStream_t s);
 void launch_mv2_partials(float4 const* vel, unsigned n, double* partials, hipStream_t s);
+// the finalize kick and the partials of the kicked velocities (the sums of
+// launch_mv2_partials, in the same order)
+void launch_finalize_mv2(float4* vel, float4 const* force, unsigned n, float half_dt, double* partials, hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Hilbert sort and particle rearrangement (hilbert.hip)

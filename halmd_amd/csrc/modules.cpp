@@ -169,7 +169,15 @@ void particle::upload_hilo(dbuf<float4>& b, double const* in, bool) {
     sync();
 }
 
+void particle::settle_thermostat() {
+    if (!owed_thermostat) return;
+    auto const owed = std::move(owed_thermostat);
+    owed_thermostat = nullptr;
+    owed();
+}
+
 void particle::settle_velocity() {
+    settle_thermostat();
     if (pending_half_dt == 0) return;
     // the kick is owed with the force of the current positions: evaluate it
     // first if it is not yet (with en_pot and stress if they were requested
@@ -222,6 +230,7 @@ void particle::get_velocity_parts(float* parts) {
     download_parts(vel, parts);
 }
 void particle::set_velocity_parts(float const* parts) {
+    settle_thermostat();   // (its chain moves on all the same)
     pending_half_dt = 0;   // overwritten
     upload_parts(vel, parts);
     velocities_changed();
@@ -238,6 +247,7 @@ void particle::get_position(double* r) {
     download_hilo(pos, r);
 }
 void particle::set_velocity(double const* v) {
+    settle_thermostat();   // (its chain moves on all the same)
     pending_half_dt = 0;   // overwritten
     upload_hilo(vel, v, false);
     velocities_changed();
@@ -421,6 +431,7 @@ void particle::evaluate_forces() {
 
 void particle::rearrange_merged(merge_scratch const& m, uint32_t* offsets, uint32_t* order_offsets, uint32_t* vals,
                                 float4* r0) {
+    settle_thermostat();
     if (force_valid) settle_velocity();   // as below
     rearrange_arrays const a{pos,     vel,     image,     id,     posq,     pos_alt,    vel_alt,
                              image_alt, id_alt, posq_alt, reverse_id, r0};
@@ -432,6 +443,7 @@ void particle::rearrange(uint32_t const* perm, float4* r0) {
     // a kick owed with a force not yet evaluated stays owed (the force will be
     // evaluated in the new order); one whose force is in memory is applied,
     // since the force array is not permuted
+    settle_thermostat();
     if (force_valid) settle_velocity();
     launch_rearrange(pos, vel, image, id, posq, perm, n, pos_alt, vel_alt, image_alt, id_alt, posq_alt, stream,
                      reverse_id, r0);
@@ -1592,14 +1604,15 @@ void verlet::set_timestep(double dt_) {
     ip.half_dt = float(dt / 2);
 }
 
-void verlet::integrate_kernel(double const* scale) {
+void verlet::integrate_kernel(double const* scale, andersen_step const* bath) {
+    p.settle_thermostat();   // another integrator's
     // plain NVE with the force of the current positions not yet evaluated and
     // a single pair force: the force kernel integrates each particle as it
     // finishes it (no separate integrate pass, no force array round trip)
     // (the owed force of the previous step is the plain one even when en_pot or
     // the stress was requested for the next evaluation, as the step that
     // evaluates its force at once computes it before any such request)
-    if (!scale && p.fused_step && fused_disp && !p.force_valid && p.forces.size() == 1 &&
+    if (!scale && !bath && p.fused_step && fused_disp && !p.force_valid && p.forces.size() == 1 &&
         (p.force_owed ? !p.owed_aux : !p.aux_enabled))
         if (p.forces[0]->integrate_fused(*this)) return;
     if (p.force_owed && !p.force_valid)
@@ -1616,7 +1629,8 @@ void verlet::integrate_kernel(double const* scale) {
     }
     float const pre = p.take_pending_kick();
     timer_integrate.start(p.stream);
-    launch_verlet_integrate(p.pos, p.vel, p.force, p.image, p.posq, p.n, ip, pre, scale, r0, slot, clear, p.stream);
+    launch_verlet_integrate(p.pos, p.vel, p.force, p.image, p.posq, p.n, ip, pre, scale, r0, slot, clear, p.stream,
+                            bath);
     timer_integrate.stop(p.stream);
     p.positions_changed();
     p.velocities_changed();
@@ -1651,8 +1665,8 @@ verlet_nvt_hoover::verlet_nvt_hoover(particle& p_, box const& b_, double dt_, do
 {
     require(T > 0 && nu > 0, "verlet_nvt_hoover: temperature and resonance frequency must be positive");
     defer_finalize = false;
-    st.resize(1);
-    partials.resize(REDUCE_BLOCKS);
+    ch->st.resize(1);
+    ch->partials.resize(REDUCE_BLOCKS);
     nhc_state s0;
     std::memset(&s0, 0, sizeof(s0));
     s0.timestep = dt_;
@@ -1662,12 +1676,13 @@ verlet_nvt_hoover::verlet_nvt_hoover(particle& p_, box const& b_, double dt_, do
 }
 
 void verlet_nvt_hoover::upload_state(nhc_state const& s) {
-    st.upload(&s, 1, p.stream);
+    ch->st.upload(&s, 1, p.stream);
     p.sync();
 }
 
 void verlet_nvt_hoover::get_state(nhc_state& out) {
-    st.download(&out, 1, p.stream);
+    if (ch->owed) p.settle_thermostat();
+    ch->st.download(&out, 1, p.stream);
     p.sync();
 }
 
@@ -1686,7 +1701,7 @@ void verlet_nvt_hoover::set_temperature(double T) {
 
 void verlet_nvt_hoover::set_timestep(double dt_) {
     verlet::set_timestep(dt_);
-    if (st.size()) {
+    if (ch->st.size()) {
         nhc_state s;
         get_state(s);
         s.timestep = dt_;
@@ -1710,19 +1725,34 @@ void verlet_nvt_hoover::set_chain(double const* xi, double const* v_xi) {
 }
 
 void verlet_nvt_hoover::integrate() {
-    p.update_force();
-    p.settle_velocity();
-    launch_mv2_partials(p.vel, p.n, partials, p.stream);
-    launch_nhc_propagate(partials, st, p.stream);
-    integrate_kernel(&st.get()->scale);
+    p.update_force();   // (a sort or rebuild that moves the particles settles first)
+    if (ch->owed) {
+        // both half steps of the chain, from the partial sums of finalize, and
+        // both rescalings in the integrate kernel
+        p.owed_thermostat = nullptr;
+        ch->owed = false;
+        launch_nhc_propagate(ch->partials, ch->st, true, p.stream);
+    } else {
+        p.settle_velocity();
+        launch_mv2_partials(p.vel, p.n, ch->partials, p.stream);
+        launch_nhc_propagate(ch->partials, ch->st, false, p.stream);
+    }
+    integrate_kernel(&ch->st.get()->scale);
 }
 
 void verlet_nvt_hoover::finalize() {
-    verlet::finalize();
-    launch_mv2_partials(p.vel, p.n, partials, p.stream);
-    launch_nhc_propagate(partials, st, p.stream);
-    launch_rescale_velocity(p.vel, p.n, &st.get()->scale, p.stream);
+    p.update_force();
+    p.settle_velocity();
+    timer_finalize.start(p.stream);
+    launch_finalize_mv2(p.vel, p.force, p.n, ip.half_dt, ch->partials, p.stream);
+    timer_finalize.stop(p.stream);
     p.velocities_changed();
+    ch->owed = true;
+    p.owed_thermostat = [c = ch, &p = p] {
+        c->owed = false;
+        launch_nhc_propagate(c->partials, c->st, false, p.stream);
+        launch_rescale_velocity(p.vel, p.n, &c->st.get()->scale, p.stream);
+    };
 }
 
 double verlet_nvt_hoover::internal_energy() {
@@ -1738,14 +1768,29 @@ verlet_nvt_andersen::verlet_nvt_andersen(particle& p_, box const& b_, uint64_t s
     require(T > 0 && rate_ >= 0, "verlet_nvt_andersen: invalid temperature or collision rate");
 }
 
+void verlet_nvt_andersen::integrate() {
+    if (last->owed) p.update_force();   // (settles first if the force was not valid any more)
+    if (!last->owed) {
+        integrate_kernel(nullptr);
+        return;
+    }
+    p.owed_thermostat = nullptr;
+    last->owed = false;
+    last->t.id = p.id;
+    integrate_kernel(nullptr, &last->t);
+}
+
 void verlet_nvt_andersen::finalize() {
     p.update_force();
     p.settle_velocity();
-    timer_finalize.start(p.stream);
-    launch_andersen_finalize(p.vel, p.force, p.id, p.n, ip.half_dt, float(rate * dt), float(std::sqrt(temperature)),
-                             seed, step++, p.stream);
-    timer_finalize.stop(p.stream);
     p.velocities_changed();
+    last->t = {nullptr, ip.half_dt, float(rate * dt), float(std::sqrt(temperature)), seed, step++};
+    last->owed = true;
+    p.owed_thermostat = [o = last, &p = p] {
+        o->owed = false;
+        o->t.id = p.id;
+        launch_andersen_finalize(p.vel, p.force, p.n, o->t, p.stream);
+    };
 }
 
 // ---------------------------------------------------------------------------

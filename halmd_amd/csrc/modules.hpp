@@ -131,7 +131,11 @@ public:
     // pass fewer); any reader of the velocities, or of the force it refers to,
     // settles it first.  0 = none pending.
     float pending_half_dt = 0;
+    // the work that a thermostat still owes the velocities (empty: none); done
+    // by settle_velocity, or taken over by that thermostat's next half step
+    std::function<void()> owed_thermostat;
     void settle_velocity();
+    void settle_thermostat();
     float take_pending_kick() { float const h = pending_half_dt; pending_half_dt = 0; return h; }
     // recompute the fixed-point snapshot after a host-side change of pos
     void download_parts(dbuf<float4> const& b, float* out);
@@ -530,15 +534,23 @@ public:
     // NVE Verlet; the thermostats need the kicked velocities at once)
     bool defer_finalize = true;
 protected:
-    void integrate_kernel(double const* scale);
+    void integrate_kernel(double const* scale, andersen_step const* bath = nullptr);
 };
 
 class verlet_nvt_hoover : public verlet {
 public:
     verlet_nvt_hoover(particle& p, box const& b, double dt, double temperature, double resonance_frequency);
     double temperature, resonance_frequency;
-    dbuf<nhc_state> st;
-    dbuf<double> partials;
+    // the chain half step and the rescaling that end a step are done together
+    // with the ones that begin the next; a reader or writer of the velocities
+    // or of the chain in between settles them (particle::owed_thermostat, which
+    // shares the chain: it outlives an integrator that is replaced)
+    struct chain {
+        dbuf<nhc_state> st;
+        dbuf<double> partials;
+        bool owed = false;
+    };
+    std::shared_ptr<chain> ch = std::make_shared<chain>();
     void set_temperature(double T);
     void set_timestep(double dt_) override;
     void set_mass(double const* m);
@@ -556,7 +568,17 @@ public:
     verlet_nvt_andersen(particle& p, box const& b, uint64_t seed, double dt, double temperature, double rate);
     uint64_t seed, step = 0;
     double temperature, rate;
+    void integrate() override;
     void finalize() override;
+private:
+    // the finalize of a step, done with the integrate of the next one, or when
+    // the velocities or the force are needed in between (particle::owed_thermostat,
+    // which shares it)
+    struct owed_step {
+        andersen_step t{};
+        bool owed = false;
+    };
+    std::shared_ptr<owed_step> last = std::make_shared<owed_step>();
 };
 
 class hilbert {

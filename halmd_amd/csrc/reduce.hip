@@ -65,14 +65,28 @@ __global__ __launch_bounds__(REDUCE_THREADS) void thermo_partials_kernel(
     block_store<THERMO_NQ>(acc, partials);
 }
 
-__global__ __launch_bounds__(REDUCE_THREADS) void mv2_partials_kernel(float4 const* __restrict__ vel, unsigned n,
-                                                                      double* __restrict__ partials) {
+// KICK: the finalize kick of verlet_finalize_kernel first.  One pass over the
+// velocities for the kick and the sum that the thermostat takes of them.
+template <bool KICK>
+__global__ __launch_bounds__(REDUCE_THREADS) void mv2_partials_kernel(typename std::conditional<KICK, float4, float4 const>::type* __restrict__ vel,
+                                                                      float4 const* __restrict__ force, float half_dt,
+                                                                      unsigned n, double* __restrict__ partials) {
     double acc[1] = {0};
     for (unsigned i = blockIdx.x * REDUCE_THREADS + threadIdx.x; i < n; i += REDUCE_BLOCKS * REDUCE_THREADS) {
         float4 const vh = vel[2 * size_t(i)], vl = vel[2 * size_t(i) + 1];
-        double const vx = double(vh.x) + double(vl.x);
-        double const vy = double(vh.y) + double(vl.y);
-        double const vz = double(vh.z) + double(vl.z);
+        ff x{vh.x, vl.x}, y{vh.y, vl.y}, z{vh.z, vl.z};
+        if constexpr (KICK) {
+            float4 const f = force[i];
+            float const k = half_dt / vh.w;
+            x = ff_add_f(x, f.x * k);
+            y = ff_add_f(y, f.y * k);
+            z = ff_add_f(z, f.z * k);
+            vel[2 * size_t(i)] = make_float4(x.hi, y.hi, z.hi, vh.w);
+            vel[2 * size_t(i) + 1] = make_float4(x.lo, y.lo, z.lo, 0.0f);
+        }
+        double const vx = double(x.hi) + double(x.lo);
+        double const vy = double(y.hi) + double(y.lo);
+        double const vz = double(z.hi) + double(z.lo);
         acc[0] += double(vh.w) * (vx * vx + vy * vy + vz * vz);
     }
     block_store<1>(acc, partials);
@@ -100,33 +114,39 @@ __global__ __launch_bounds__(REDUCE_THREADS) void reduce_final_kernel(double con
 
 // Nose-Hoover chain of length 2, half step (Martyna et al., J. Chem. Phys. 97,
 // 2635 (1992)); operation order of halmd/mdsim/gpu/integrators/verlet_nvt_hoover.cpp:188-222
+// half steps: 1, or 2 with the velocities rescaled in between
 __global__ __launch_bounds__(REDUCE_THREADS) void nhc_propagate_kernel(double const* __restrict__ partials,
-                                                                       nhc_state* __restrict__ st) {
+                                                                       nhc_state* __restrict__ st, int half_steps) {
     double en_kin_2 = sum_partials(partials, 1, 0);
     if (threadIdx.x != 0) return;
     double const T = st->temperature, target = st->en_kin_target_2;
     double const dt2 = st->timestep / 2, dt4 = st->timestep / 4, dt8 = st->timestep / 8;
     double const m0 = st->mass_xi[0], m1 = st->mass_xi[1];
-    double v0 = st->v_xi[0], v1 = st->v_xi[1];
-    v1 += (m0 * v0 * v0 - T) / m1 * dt4;
-    double const t = exp(-v1 * dt8);
-    v0 *= t;
-    v0 += (en_kin_2 - target) / m0 * dt4;
-    v0 *= t;
-    st->xi[0] += v0 * dt2;
-    st->xi[1] += v1 * dt2;
-    double const s = exp(-v0 * dt2);
-    en_kin_2 *= s * s;
-    v0 *= t;
-    v0 += (en_kin_2 - target) / m0 * dt4;
-    v0 *= t;
-    v1 += (m0 * v0 * v0 - T) / m1 * dt4;
+    double v0 = st->v_xi[0], v1 = st->v_xi[1], x0 = st->xi[0], x1 = st->xi[1], scale = 1;
+    for (int h = 0; h < half_steps; ++h) {
+        v1 += (m0 * v0 * v0 - T) / m1 * dt4;
+        double const t = exp(-v1 * dt8);
+        v0 *= t;
+        v0 += (en_kin_2 - target) / m0 * dt4;
+        v0 *= t;
+        x0 += v0 * dt2;
+        x1 += v1 * dt2;
+        double const s = exp(-v0 * dt2);
+        en_kin_2 *= s * s;   // (the sum of the rescaled velocities, to their rounding)
+        v0 *= t;
+        v0 += (en_kin_2 - target) / m0 * dt4;
+        v0 *= t;
+        v1 += (m0 * v0 * v0 - T) / m1 * dt4;
+        scale *= s;
+    }
+    st->xi[0] = x0;
+    st->xi[1] = x1;
     st->v_xi[0] = v0;
     st->v_xi[1] = v1;
-    st->scale = s;
+    st->scale = scale;
     // extended-energy contribution, divided by N on the host
     double const dN = target / T;
-    st->en_nhc_raw = T * (dN * st->xi[0] + st->xi[1]) + 0.5 * (m0 * v0 * v0 + m1 * v1 * v1);
+    st->en_nhc_raw = T * (dN * x0 + x1) + 0.5 * (m0 * v0 * v0 + m1 * v1 * v1);
 }
 
 } // namespace
@@ -144,12 +164,18 @@ void launch_reduce_final(double const* partials, unsigned nq, double* out, hipSt
 }
 
 void launch_mv2_partials(float4 const* vel, unsigned n, double* partials, hipStream_t s) {
-    mv2_partials_kernel<<<REDUCE_BLOCKS, REDUCE_THREADS, 0, s>>>(vel, n, partials);
+    mv2_partials_kernel<false><<<REDUCE_BLOCKS, REDUCE_THREADS, 0, s>>>(vel, nullptr, 0.0f, n, partials);
     HIP_CHECK(hipGetLastError());
 }
 
-void launch_nhc_propagate(double const* partials, nhc_state* state, hipStream_t s) {
-    nhc_propagate_kernel<<<1, REDUCE_THREADS, 0, s>>>(partials, state);
+void launch_finalize_mv2(float4* vel, float4 const* force, unsigned n, float half_dt, double* partials,
+                         hipStream_t s) {
+    mv2_partials_kernel<true><<<REDUCE_BLOCKS, REDUCE_THREADS, 0, s>>>(vel, force, half_dt, n, partials);
+    HIP_CHECK(hipGetLastError());
+}
+
+void launch_nhc_propagate(double const* partials, nhc_state* state, bool two, hipStream_t s) {
+    nhc_propagate_kernel<<<1, REDUCE_THREADS, 0, s>>>(partials, state, two ? 2 : 1);
     HIP_CHECK(hipGetLastError());
 }
 

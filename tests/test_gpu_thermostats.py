@@ -1,0 +1,47 @@
+"""What a thermostat leaves to the next step is done in time for every reader."""
+
+import numpy as np
+import pytest
+
+from halmd_amd import workloads
+
+pytestmark = pytest.mark.gpu
+
+OPTIONS = {"verlet_nvt_hoover": dict(resonance_frequency=5.0), "verlet_nvt_andersen": dict(collision_rate=5.0)}
+
+
+def _system(integrator, n):
+    return workloads.lennard_jones(n, density=0.8442, temperature=1.2, jitter=0.02, seed=11, timestep=0.004,
+                                   integrator=integrator, sort_interval=25, **OPTIONS[integrator])
+
+
+# (not a multiple of a wave; several workgroups; more particles than the partial
+# sums have threads)
+@pytest.mark.parametrize("n", [1001, 4096, 70000])
+@pytest.mark.parametrize("integrator", sorted(OPTIONS))
+def test_reading_between_steps_leaves_the_trajectory(integrator, n):
+    a, b = _system(integrator, n), _system(integrator, n)
+    steps = 60
+    a.sampler.run(steps)
+    for k in range(steps):
+        b.sampler.run(1)
+        if k % 3 == 0:
+            b.particle.data["velocity"]
+        elif k % 7 == 1:
+            b.particle.data["velocity"] = b.particle.data["velocity"]
+        if integrator == "verlet_nvt_hoover" and k % 5 == 0:
+            b.integrator.set_temperature(1.2)
+            b.integrator.position
+    if integrator == "verlet_nvt_andersen":
+        # the same arithmetic in either kernel
+        for name in ("position", "velocity", "image"):
+            assert np.array_equal(a.particle.ordered(name), b.particle.ordered(name)), name
+    else:
+        # the sum of the rescaled velocities is taken from the one before: FP64
+        # rounding in the scale, which can flip the last bit of a fixed-point
+        # coordinate (L / 2^32 = 1e-8); with a curvature of 1e3 and dt = 0.004
+        # that is 4e-8 in a velocity, which grows by a few e in 60 steps
+        for name in ("position", "velocity"):
+            assert np.max(np.abs(a.particle.ordered(name) - b.particle.ordered(name))) < 1e-6, name
+        assert np.allclose(a.integrator.position, b.integrator.position, rtol=1e-6, atol=1e-12)
+        assert np.allclose(a.integrator.velocity, b.integrator.velocity, rtol=1e-6, atol=1e-9)
