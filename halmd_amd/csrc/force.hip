@@ -67,6 +67,21 @@ __device__ __forceinline__ float pow_half(float x, unsigned k) {
     return r;
 }
 
+// the same for N values and a wave-uniform k: the exponent's loop and branches
+// run once for all of them
+template <int N>
+__device__ __forceinline__ void pow_half_n(float (&x)[N], unsigned k, float (&r)[N]) {
+#pragma unroll
+    for (int t = 0; t < N; ++t) r[t] = (k & 1u) ? sqrtf(x[t]) : 1.0f;
+    for (unsigned e = k >> 1; e; e >>= 1) {
+        if (e & 1u)
+#pragma unroll
+            for (int t = 0; t < N; ++t) r[t] *= x[t];
+#pragma unroll
+        for (int t = 0; t < N; ++t) x[t] *= x[t];
+    }
+}
+
 template <int KIND, int TRUNC>
 __device__ __forceinline__ void pair_eval(float rr, float morse_d, pair_param const& pp, float rri_smooth,
                                           float& fval, float& en) {
@@ -926,25 +941,29 @@ void staged_trunc(staged_launch const& a) {
 // coordinates.
 //
 // Grid: x over blocks of FULL_TILE particles i (one per lane), y over `parts`
-// contiguous ranges of j, each a multiple of FULL_TILE long, so that small
-// systems still occupy the whole chip.  Each workgroup stages its j range in
-// tiles of FULL_TILE records through LDS and every lane sums over the tile:
-// FP32 over groups of 8 pairs, Kahan over the groups.  Part y writes its sums
-// (force x, y, z, en_pot, 6 stress components) to partial[(y * 10 + c) * n1 + i];
+// contiguous ranges of j (pair_full_split), so that small systems still occupy
+// the whole chip.  Each workgroup stages its j range in tiles of FULL_TILE
+// records through LDS and every lane sums over the tile: FP32 over groups of 8
+// pairs, Kahan over the groups.  Part y writes its sums (force x, y, z, en_pot,
+// 6 stress components) to partial[(y * 10 + c) * n1 + i];
 // pair_full_reduce_kernel adds the parts in order (Kahan), scales the aux
 // sums by aux_weight and adds the stored values unless force_zero.  Both the
 // split and the order depend only on (n1, n2).
+// Bound by VALU issue.  One species (MULTI = false): the parameters live in
+// scalar registers, and the exponents of a power law are uniform, so that the
+// eight pairs of a group share the steps of the power: 6000 particles with
+// U ~ r^-12 227 -> 66 us, 63 instructions a pair.
 constexpr unsigned FULL_TILE = 256;
 constexpr unsigned FULL_COMPONENTS = PAIR_FULL_COMPONENTS;
 
-template <int KIND, bool AUX>
+template <int KIND, bool AUX, bool MULTI>
 __global__ __launch_bounds__(FULL_TILE) void pair_full_kernel(
     uint4 const* __restrict__ posq1, unsigned n1, uint4 const* __restrict__ posq2, unsigned n2, unsigned same,
     unsigned chunk, force_params P, float* __restrict__ partial)
 {
     __shared__ pair_param s_pair[MAX_TYPES * MAX_TYPES];
     __shared__ uint4 s_q[FULL_TILE];
-    if (threadIdx.x < MAX_TYPES * MAX_TYPES) s_pair[threadIdx.x] = P.pair[threadIdx.x];
+    if (MULTI && threadIdx.x < MAX_TYPES * MAX_TYPES) s_pair[threadIdx.x] = P.pair[threadIdx.x];
 
     unsigned const i = blockIdx.x * FULL_TILE + threadIdx.x;
     bool const active = i < n1;
@@ -952,44 +971,85 @@ __global__ __launch_bounds__(FULL_TILE) void pair_full_kernel(
     unsigned const ti = (qi.w & 3u) * P.ntype;
     unsigned const j0 = blockIdx.y * chunk, j1 = min(n2, j0 + chunk);
 
-    float fx = 0, fy = 0, fz = 0, cx = 0, cy = 0, cz = 0;
-    float bx = 0, by = 0, bz = 0;
-    float en = 0, ce = 0, be = 0;
-    float st[6] = {0, 0, 0, 0, 0, 0}, cs[6] = {0, 0, 0, 0, 0, 0}, bs[6] = {0, 0, 0, 0, 0, 0};
+    constexpr int NS = AUX ? 10 : 3, G = 8;
+    float b[NS] = {}, f[NS] = {}, c[NS] = {};   // group sums, Kahan sums over the groups
 
-    auto pair = [&](uint4 const qj) {
-        int32_t const Dx = int32_t(qi.x - qj.x), Dy = int32_t(qi.y - qj.y), Dz = int32_t(qi.z - qj.z);
-        float const dx = separation(Dx, P.q[0], P.q_lo[0]);
-        float const dy = separation(Dy, P.q[1], P.q_lo[1]);
-        float const dz = separation(Dz, P.q[2], P.q_lo[2]);
-        float const rr = dx * dx + dy * dy + dz * dz;
-        pair_param const& pp = s_pair[ti + (qj.w & 3u)];
-        float const md = KIND == POTENTIAL_MORSE ? morse_argument(rr, pp) : 0.0f;
-        float fval, u;
-        pair_eval<KIND, TRUNC_SHARP>(rr, md, pp, 0.0f, fval, u);
-        bx += fval * dx;
-        by += fval * dy;
-        bz += fval * dz;
-        if (AUX) {
-            be += u;
-            bs[0] += fval * dx * dx;
-            bs[1] += fval * dy * dy;
-            bs[2] += fval * dz * dz;
-            bs[3] += fval * dx * dy;
-            bs[4] += fval * dx * dz;
-            bs[5] += fval * dy * dz;
-        }
-    };
-    auto fold = [&]() {
-        kahan_add(fx, cx, bx);
-        kahan_add(fy, cy, by);
-        kahan_add(fz, cz, bz);
-        bx = by = bz = 0;
-        if (AUX) {
-            kahan_add(en, ce, be);
-            be = 0;
+    // the exponents of a uniform power law, in scalar registers
+    unsigned const em = __builtin_amdgcn_readfirstlane(unsigned(P.pair[0].p_lo[0]));
+    unsigned const en = __builtin_amdgcn_readfirstlane(unsigned(P.pair[0].p_lo[1]));
+
+    // the pairs with records k .. k + 7 of the tile; CHECK: without those from
+    // record m on and the record `self`
+    auto group = [&](auto check, unsigned k, unsigned m, unsigned self) {
+        constexpr bool CHECK = decltype(check)::value;
+        float dx[G], dy[G], dz[G], rr[G], fval[G], u[G];
+        unsigned tj[G];
 #pragma unroll
-            for (int c = 0; c < 6; ++c) { kahan_add(st[c], cs[c], bs[c]); bs[c] = 0; }
+        for (int t = 0; t < G; ++t) {
+            uint4 const qj = s_q[CHECK ? min(k + t, m - 1) : k + t];
+            int32_t const Dx = int32_t(qi.x - qj.x), Dy = int32_t(qi.y - qj.y), Dz = int32_t(qi.z - qj.z);
+            dx[t] = separation(Dx, P.q[0], P.q_lo[0]);
+            dy[t] = separation(Dy, P.q[1], P.q_lo[1]);
+            dz[t] = separation(Dz, P.q[2], P.q_lo[2]);
+            rr[t] = dx[t] * dx[t] + dy[t] * dy[t] + dz[t] * dz[t];
+            if (MULTI) tj[t] = qj.w & 3u;
+        }
+        if constexpr (KIND == POTENTIAL_POWER_LAW && !MULTI) {
+            // (pair_eval's operations)
+            pair_param const& pp = P.pair[0];
+            float rri[G], x[G], inv[G], sn[G], smn[G];
+#pragma unroll
+            for (int t = 0; t < G; ++t) {
+                if (pp.p[3] != 0.0f) {
+                    float const r = sqrtf(rr[t]);
+                    float const rs = r - pp.p[3];
+                    rri[t] = pp.p[2] * rcp_nr(rs * rs);
+                    inv[t] = rcp_nr(rs * r);
+                } else {
+                    inv[t] = rcp_nr(rr[t]);
+                    rri[t] = pp.p[2] * inv[t];
+                }
+                x[t] = rri[t];
+            }
+            pow_half_n(x, en, sn);
+            pow_half_n(rri, em - en, smn);
+#pragma unroll
+            for (int t = 0; t < G; ++t) {
+                fval[t] = sn[t] * (pp.p_lo[0] * pp.p[0] * smn[t] - pp.p_lo[1] * pp.p[1]) * inv[t];
+                u[t] = sn[t] * (pp.p[0] * smn[t] - pp.p[1]);
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < G; ++t) {
+                pair_param const& pp = MULTI ? s_pair[ti + tj[t]] : P.pair[0];
+                float const md = KIND == POTENTIAL_MORSE ? morse_argument(rr[t], pp) : 0.0f;
+                pair_eval<KIND, TRUNC_SHARP>(rr[t], md, pp, 0.0f, fval[t], u[t]);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < G; ++t) {
+            if (CHECK) {
+                bool const use = k + t < m && k + t != self;
+                fval[t] = use ? fval[t] : 0.0f;
+                u[t] = use ? u[t] : 0.0f;
+            }
+            b[0] += fval[t] * dx[t];
+            b[1] += fval[t] * dy[t];
+            b[2] += fval[t] * dz[t];
+            if constexpr (AUX) {
+                b[3] += u[t];
+                b[4] += fval[t] * dx[t] * dx[t];
+                b[5] += fval[t] * dy[t] * dy[t];
+                b[6] += fval[t] * dz[t] * dz[t];
+                b[7] += fval[t] * dx[t] * dy[t];
+                b[8] += fval[t] * dx[t] * dz[t];
+                b[9] += fval[t] * dy[t] * dz[t];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            kahan_add(f[k], c[k], b[k]);
+            b[k] = 0;
         }
     };
 
@@ -1000,35 +1060,16 @@ __global__ __launch_bounds__(FULL_TILE) void pair_full_kernel(
         __syncthreads();
         if (!active) continue;
         // the tile holding j = i (same instance) takes the per-pair test
-        bool const self = same && i >= jt && i < jt + m;
+        unsigned const self = same && i >= jt && i < jt + m ? i - jt : ~0u;
         unsigned k = 0;
-        for (; k + 8 <= m; k += 8) {
-            if (self) {
-#pragma unroll
-                for (unsigned t = 0; t < 8; ++t)
-                    if (jt + k + t != i) pair(s_q[k + t]);
-            } else {
-#pragma unroll
-                for (unsigned t = 0; t < 8; ++t) pair(s_q[k + t]);
-            }
-            fold();
-        }
-        if (k < m) {
-            for (; k < m; ++k)
-                if (!self || jt + k != i) pair(s_q[k]);
-            fold();
-        }
+        if (self == ~0u)
+            for (; k + G <= m; k += G) group(std::false_type{}, k, m, self);
+        for (; k < m; k += G) group(std::true_type{}, k, m, self);
     }
     if (!active) return;
     size_t const base = size_t(blockIdx.y) * FULL_COMPONENTS * n1 + i;
-    partial[base] = fx - cx;
-    partial[base + n1] = fy - cy;
-    partial[base + 2 * size_t(n1)] = fz - cz;
-    if (AUX) {
-        partial[base + 3 * size_t(n1)] = en - ce;
 #pragma unroll
-        for (int c = 0; c < 6; ++c) partial[base + (4 + c) * size_t(n1)] = st[c] - cs[c];
-    }
+    for (int k = 0; k < NS; ++k) partial[base + k * size_t(n1)] = f[k] - c[k];
 }
 
 template <bool AUX>
@@ -1042,6 +1083,8 @@ __global__ __launch_bounds__(256) void pair_full_reduce_kernel(
     float s[NC], c[NC];
 #pragma unroll
     for (unsigned k = 0; k < NC; ++k) s[k] = c[k] = 0;
+    // (few waves: the loads of eight parts in flight)
+#pragma unroll 8
     for (unsigned y = 0; y < parts; ++y) {
         size_t const base = size_t(y) * FULL_COMPONENTS * n1 + i;
 #pragma unroll
@@ -1073,10 +1116,13 @@ template <int KIND>
 void pair_full_go(uint4 const* posq1, unsigned n1, uint4 const* posq2, unsigned n2, bool same, unsigned parts,
                   unsigned chunk, force_params const& p, bool aux, float* partial, hipStream_t s) {
     dim3 const grid((n1 + FULL_TILE - 1) / FULL_TILE, parts);
-    if (aux)
-        pair_full_kernel<KIND, true><<<grid, FULL_TILE, 0, s>>>(posq1, n1, posq2, n2, same, chunk, p, partial);
+    auto const go = [&](auto kernel) {
+        kernel<<<grid, FULL_TILE, 0, s>>>(posq1, n1, posq2, n2, same, chunk, p, partial);
+    };
+    if (p.ntype > 1)
+        aux ? go(pair_full_kernel<KIND, true, true>) : go(pair_full_kernel<KIND, false, true>);
     else
-        pair_full_kernel<KIND, false><<<grid, FULL_TILE, 0, s>>>(posq1, n1, posq2, n2, same, chunk, p, partial);
+        aux ? go(pair_full_kernel<KIND, true, false>) : go(pair_full_kernel<KIND, false, false>);
 }
 } // namespace
 
@@ -1104,14 +1150,28 @@ void launch_pair_force(uint4 const* posq, unsigned n, uint32_t const* list, uint
 }
 
 namespace {
-// the j ranges of launch_pair_full: chunk (a multiple of FULL_TILE) and their
-// number; about 512 workgroups (2048 waves) for small n1
+// The j ranges of launch_pair_full: chunk (a multiple of 64) and their number.
+// The time is that of the compute unit with the most workgroups: its rounds of
+// chunk + 16 pairs (16: staging, start and end of a workgroup), and 1 for each
+// part that the reduction adds.  N = 6000 in 24 blocks: 32 parts of 192, three
+// workgroups for each unit, where 12 parts of 512 left most units one and some
+// two.
 void pair_full_split(unsigned n1, unsigned n2, unsigned& chunk, unsigned& parts) {
-    unsigned const blocks = std::max(1u, (n1 + FULL_TILE - 1) / FULL_TILE);
-    unsigned const tiles = (n2 + FULL_TILE - 1) / FULL_TILE;
-    unsigned const want = std::max(1u, std::min({(512 + blocks - 1) / blocks, tiles, PAIR_FULL_MAX_PARTS}));
-    chunk = ((tiles + want - 1) / want) * FULL_TILE;
-    parts = n2 ? (n2 + chunk - 1) / chunk : 0;
+    constexpr unsigned UNITS = 256, STEP = 64;
+    uint64_t const blocks = std::max(1u, (n1 + FULL_TILE - 1) / FULL_TILE);
+    uint64_t best = ~uint64_t(0);
+    chunk = STEP;
+    parts = 0;
+    for (unsigned want = 1; n2 && want <= PAIR_FULL_MAX_PARTS; ++want) {
+        unsigned const c = (((n2 + want - 1) / want + STEP - 1) / STEP) * STEP, np = (n2 + c - 1) / c;
+        if (np != want) continue;   // (seen, or to be seen, as its own)
+        uint64_t const cost = (blocks * np + UNITS - 1) / UNITS * (c + 16) + np;
+        if (cost < best) {
+            best = cost;
+            chunk = c;
+            parts = np;
+        }
+    }
 }
 } // namespace
 

@@ -78,6 +78,25 @@ def test_pair_full_matches_fp64(oracle, kind, n):
     assert np.all(np.abs(f.sum(axis=0)) < 1e-5 * rms * np.sqrt(n))
 
 
+@pytest.mark.parametrize("index,n", [(12, 2), (7, 65), (48, 257), (12, 1000), (9, 1601)])
+def test_pair_full_power_law_sizes(oracle, index, n):
+    # one species, exponents odd and even: groups of 8 pairs, the tile of the
+    # particle itself, tiles and parts that end anywhere
+    L, r0, species = _system(n, 0.8, "power_law", seed=n)
+    p = mdsim.particle(particles=n, species=1)
+    p.data["position"] = r0
+    pot = mdsim.potentials.pair.power_law(epsilon=1.0, sigma=0.9, index=index)
+    force = mdsim.forces.pair(box=mdsim.box(length=L), particle=p, potential=pot)
+    assert isinstance(force, mdsim.forces.pair_full)
+    f, u = p.data["force"], p.data["potential_energy"]
+    fref, uref, _ = oracle.pair_force_brute(
+        r0, species, L, oracle.Potential(oracle.POT_POWER_LAW, "sharp", 1.0, 0.9, NO_CUTOFF, index=index))
+    # the fixed-point coordinates (L / 2^33) enter a force of the closest pair
+    # index + 2 times, and each of the power's steps rounds once more
+    assert _force_error(f, fref) < FORCE_TOL * (index + 2) / 14
+    assert abs(u.sum() - uref.sum()) / abs(uref.sum()) < AUX_TOL * (index + 2) / 14
+
+
 def test_pair_full_two_instances(oracle):
     # force on instance 1 from every particle of instance 2 = (force on 1 in
     # the union) - (force on 1 from itself); moving instance 2 invalidates it
