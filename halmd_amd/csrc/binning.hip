@@ -228,7 +228,8 @@ __global__ __launch_bounds__(256) void build_all_pairs_kernel(uint4 const* __res
     unsigned const lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE;
     unsigned const i0 = blockIdx.x * AP_PER_GROUP;
     if (cond.slots) {
-        if (!displacement_aborts(displacement_word(cond.slots), cond.slots, cond.keep_bits)) return;   // the whole workgroup
+        // the whole workgroup
+        if (!displacement_aborts(displacement_word(cond.slots), cond.slots, cond.keep_bits)) return;
         if (threadIdx.x < AP_PER_GROUP && i0 + threadIdx.x < n)
             cond.r0[i0 + threadIdx.x] = cond.pos[2 * size_t(i0 + threadIdx.x)];
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(cond.rebuilt, 1u);
@@ -604,7 +605,7 @@ __device__ __forceinline__ void staged_build_segment(
 }
 
 template <bool MULTI, bool ISO, bool FOLD, unsigned SPLIT>
-__global__ __launch_bounds__(SEG_THREADS_MAX) void build_staged_kernel(
+__global__ __launch_bounds__(SPLIT ? SPLIT * SPLIT_WAVES * WAVE : SEG_THREADS_MAX) void build_staged_kernel(
     uint4 const* __restrict__ posq, uint32_t const* __restrict__ off, seg_params sp, neighbour_params p,
     unsigned cap, uint16_t* __restrict__ list, uint32_t* __restrict__ count, uint32_t* __restrict__ stats)
 {
@@ -793,7 +794,8 @@ __global__ __launch_bounds__(SEG_THREADS_MAX) void build_windowed_kernel(
 
     unsigned const seg = seg_of_block(sp, blockIdx.x);
     if (seg >= sp.nseg) return;   // the whole workgroup
-    windowed_build_segment<MULTI>(posq, off, soff, sp, seg, p, cap, list, count, stat_pair(stats), s_rec, st, s_bound, s_rr,
+    windowed_build_segment<MULTI>(posq, off, soff, sp, seg, p, cap, list, count, stat_pair(stats), s_rec, st, s_bound,
+                                  s_rr,
                                   s_yz);
 }
 
@@ -1589,14 +1591,22 @@ void launch_build_neighbours_staged(uint4 const* posq, unsigned n, uint32_t cons
     }
     size_t const bounds = size_t(3) * (sp.R + 2) * (sp.S + 3) * sizeof(unsigned);
     size_t const lds = size_t(sp.lds_cap) * (p.iso ? sizeof(uint2) : sizeof(uint4)) + bounds;
-    bool const split = n < BUILD_SPLIT_BELOW && lds + sizeof(build_stage<1>) + BUILD_TABLES <= BUILD_LDS_MAX;
+    // groups of three waves: two where a segment holds more than 64 particles (a
+    // second pass over one group's waves costs more than the split gains: 44
+    // against 58 us at N = 64,000 with 93 a segment, 61 against 79 us for a slab
+    // of 100,003 with 99)
+    auto const fits = [&](size_t stage) { return lds + stage + BUILD_TABLES <= BUILD_LDS_MAX; };
+    unsigned groups = n >= BUILD_SPLIT_BELOW ? 0 : div_up(n, sp.nseg) <= WAVE ? 1 : 2;
+    if (groups == 2 && !fits(sizeof(build_stage<2>))) groups = 0;
+    if (groups == 1 && !fits(sizeof(build_stage<1>))) groups = 0;
     bool const fold = p.ntype == 1 && p.iso && std::min({sp.grid.ncell[0], sp.grid.ncell[1], sp.grid.ncell[2]}) >= 5;
     auto const go = [&](auto kernel, unsigned threads) {
         kernel<<<grid, threads, lds, s>>>(posq, offset, sp, p, cap, list, count, stats);
     };
 #define HALMD_BUILD_STAGED(...)                                                                                       \
-    (split ? go(build_staged_kernel<__VA_ARGS__, 1>, SPLIT_WAVES * WAVE)                                           \
-           : go(build_staged_kernel<__VA_ARGS__, 0>, sp.threads))
+    (groups == 2   ? go(build_staged_kernel<__VA_ARGS__, 2>, 2 * SPLIT_WAVES * WAVE)                                  \
+     : groups == 1 ? go(build_staged_kernel<__VA_ARGS__, 1>, SPLIT_WAVES * WAVE)                                      \
+                   : go(build_staged_kernel<__VA_ARGS__, 0>, sp.threads))
     if (p.ntype > 1) {
         if (p.iso) HALMD_BUILD_STAGED(true, true, false);
         else HALMD_BUILD_STAGED(true, false, false);

@@ -1208,8 +1208,9 @@ void launch_pair_full(uint4 const* posq1, unsigned n1, uint4 const* posq2, unsig
 }
 
 void launch_pair_force_staged(uint4 const* posq, unsigned n, uint32_t const* offset, seg_params const& sp,
-                              uint16_t const* list, uint32_t const* count, unsigned cap, force_params const& p, bool aux, bool force_zero,
-                              float aux_weight, float4* force, float* stress, unsigned stride, hipStream_t s,
+                              uint16_t const* list, uint32_t const* count, unsigned cap, force_params const& p,
+                              bool aux, bool force_zero, float aux_weight, float4* force, float* stress,
+                              unsigned stride, hipStream_t s,
                               displacement_check const* check, fused_integrate const* fuse) {
     if (!sp.nseg) return;
     if (fuse && aux) throw error(HALMD_ERR_INVALID_ARGUMENT, "pair force: the fused step has no aux path");

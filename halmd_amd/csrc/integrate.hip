@@ -66,7 +66,7 @@ __device__ __forceinline__ void andersen_kick(andersen_step const& t, uint32_t i
 }
 
 // ANDERSEN: the previous step's finalize first (andersen_kick), a pass over the
-// velocities and forces less: 4.0 us for both at N = 10,007, 3.5 + 3.5 apart
+// velocities and forces less: 4.5 us for both at N = 10,007, 3.6 + 3.5 apart
 template <bool ANDERSEN>
 __global__ __launch_bounds__(256) void verlet_integrate_kernel(
     float4* __restrict__ pos, float4* __restrict__ vel, float4 const* __restrict__ force, int4* __restrict__ image,

@@ -235,18 +235,10 @@ __host__ __device__ inline size_t list16_index(size_t i, size_t k, size_t cap) {
 }
 constexpr unsigned STAT_SLOTS = 64, STAT_STRIDE = 32;   // (128 bytes apart)
 // Single systems below BUILD_SPLIT_BELOW particles build their lists by three
-// waves per 64 particles: 27 against 48 us at N = 4000, 43 against 64 us at
-// N = 64,000, 63 us either way at N = 108,000, 210 against 146 us at N = 524,288.
-constexpr unsigned BUILD_SPLIT_BELOW = 1u << 17;
-// Lists are padded with the slot U of a sentinel record (staged after the
-// union, at least a third of the box away from every particle of the segment
-// in y and z) to a multiple of 8 entries; count[i] excludes the padding.
-// stats: STAT_SLOTS pairs of words STAT_STRIDE apart, whose largest values are
-// the largest count (may exceed cap) and the largest staging size U + 1 (a
-// segment whose staging exceeds sp.lds_cap builds nothing; the caller retries).
-// Workgroup b raises pair b % STAT_SLOTS: atomics on one word take about 15 ns
-// each on this chip whatever else it does, and the 23,000 of a build at N =
-// 2^20 on one word took all of its 370 us.
+// waves per 64 particles: 27 against 48 us at N = 4000, 31 against 54 at 32,000,
+// 44 against 65 at 64,000, 61 against 69 for a slab of 100,003; 73 against 70 at
+// 108,000, 210 against 146 us at N = 524,288.
+constexpr unsigned BUILD_SPLIT_BELOW = 104 * 1024;
 //
 // With sub_offset (the offsets of the (cell, x sub-bin) order the particles
 // are in, ncells SUB_BINS + 1 entries; cubic box, nx >= 4) each lane scans

@@ -1515,8 +1515,8 @@ bool pair_trunc::launch(bool force_zero, displacement_check const* check, fused_
     }
     timer.start(p.stream);
     if (nb.staged)
-        launch_pair_force_staged(p.posq, p.n, nb.bin->order_offset, nb.sp_force, nb.list16, nb.count, nb.cap, params, aux,
-                                 force_zero, w, p.force, p.stress, p.n_pad, p.stream, check, fuse);
+        launch_pair_force_staged(p.posq, p.n, nb.bin->order_offset, nb.sp_force, nb.list16, nb.count, nb.cap, params,
+                                 aux, force_zero, w, p.force, p.stress, p.n_pad, p.stream, check, fuse);
     else
         launch_pair_force(p.posq, p.n, nb.list, nb.count, nb.cap, params, aux, force_zero, w, p.force, p.stress,
                           p.n_pad, p.stream, fuse, p2.posq);

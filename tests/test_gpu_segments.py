@@ -18,8 +18,8 @@ def _system(kind, n, jitter):
 
 
 # 4 cells a side, some particles more than whole waves, two species; either side
-# of the limit of the list build by three waves (2^17)
-@pytest.mark.parametrize("kind,n", [("lj", 1372), ("lj", 4001), ("ka", 8788), ("lj", 131071), ("lj", 131072)])
+# of the limit of the list build by three waves (104 * 1024)
+@pytest.mark.parametrize("kind,n", [("lj", 1372), ("lj", 4001), ("ka", 8788), ("lj", 106495), ("lj", 106496)])
 def test_shape_leaves_lists(oracle, kind, n):
     w = _system(kind, n, 0.15)
     for shape in SHAPES:
