@@ -1151,22 +1151,28 @@ void launch_pair_force(uint4 const* posq, unsigned n, uint32_t const* list, uint
 
 namespace {
 // The j ranges of launch_pair_full: chunk (a multiple of 64) and their number.
-// The time is that of the compute unit with the most workgroups: its rounds of
-// chunk + 16 pairs (16: staging, start and end of a workgroup), and 1 for each
-// part that the reduction adds.  N = 6000 in 24 blocks: 32 parts of 192, three
-// workgroups for each unit, where 12 parts of 512 left most units one and some
-// two.
+// The time is that of the compute unit with the most workgroups, W: their
+// pairs, W (chunk + 16) (16: staging, start and end of a workgroup), and once
+// more those of one, since W waves a SIMD hide all but 1 / (W + 1) of a wave's
+// latency; and 1 for each part that the reduction adds.  W = 1, 2, 4, 8 at N =
+// 65,536 with two species: 3023, 2030, 1800, 1665 us a step (1555 at 48), with one
+// species and U ~ r^-12 8375, 5140, 4411, 4022 us (3681).  Of eleven splits at each
+// of 13 sizes from 600 to 65,536 this one is within 10% of the fastest.
+// More parts have to be 3% faster, for their scratch, which is bounded by
+// PAIR_FULL_MAX_BYTES.
 void pair_full_split(unsigned n1, unsigned n2, unsigned& chunk, unsigned& parts) {
     constexpr unsigned UNITS = 256, STEP = 64;
     uint64_t const blocks = std::max(1u, (n1 + FULL_TILE - 1) / FULL_TILE);
+    uint64_t const part_bytes = PAIR_FULL_COMPONENTS * sizeof(float) * uint64_t(n1);
     uint64_t best = ~uint64_t(0);
     chunk = STEP;
     parts = 0;
     for (unsigned want = 1; n2 && want <= PAIR_FULL_MAX_PARTS; ++want) {
+        if (want > 1 && want * part_bytes > PAIR_FULL_MAX_BYTES) break;
         unsigned const c = (((n2 + want - 1) / want + STEP - 1) / STEP) * STEP, np = (n2 + c - 1) / c;
         if (np != want) continue;   // (seen, or to be seen, as its own)
-        uint64_t const cost = (blocks * np + UNITS - 1) / UNITS * (c + 16) + np;
-        if (cost < best) {
+        uint64_t const cost = ((blocks * np + UNITS - 1) / UNITS + 1) * (c + 16) + np;
+        if (best == ~uint64_t(0) || cost < best - best / 32) {
             best = cost;
             chunk = c;
             parts = np;

@@ -296,9 +296,11 @@ void launch_pair_force(uint4 const* posq, unsigned n, uint32_t const* list, uint
 // untruncated forces over all pairs of two particle instances (same: one
 // instance, j != i); p as from potential::device_params for pair_full (sharp,
 // infinite cutoff).  partial: pair_full_partial_floats(n1, n2) floats of
-// scratch, at most PAIR_FULL_MAX_PARTS * PAIR_FULL_COMPONENTS * n1.
+// scratch, PAIR_FULL_COMPONENTS * n1 for each of at most PAIR_FULL_MAX_PARTS
+// parts (one part, or PAIR_FULL_MAX_BYTES at most).
 constexpr unsigned PAIR_FULL_MAX_PARTS = 64;
 constexpr unsigned PAIR_FULL_COMPONENTS = 10;
+constexpr size_t PAIR_FULL_MAX_BYTES = size_t(64) << 20;
 size_t pair_full_partial_floats(unsigned n1, unsigned n2);
 void launch_pair_full(uint4 const* posq1, unsigned n1, uint4 const* posq2, unsigned n2, bool same,
                       force_params const& p, bool aux, bool force_zero, float aux_weight, float4* force,

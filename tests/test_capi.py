@@ -205,3 +205,24 @@ def test_skin_per_potential():
     for sp in specs:
         assert spec_skin(0.3, sp) == 0.3
         assert spec_skin(skins, sp) == skins[sp["potential"]]
+
+
+def test_pair_full_scratch_and_workgroups():
+    # the parts that the all-pairs force splits its sums into (10 floats a
+    # particle and part): scratch of at most 64 MiB, or one part; at least two
+    # workgroups of 256 particles for each of the 256 compute units where the
+    # parts (64 particles long at least) and the scratch allow it
+    floats = _lib.lib()["_ZN5halmd24pair_full_partial_floatsEjj"]
+    floats.restype, floats.argtypes = ctypes.c_size_t, [ctypes.c_uint, ctypes.c_uint]
+    assert floats(1000, 0) == 0
+    for n in [2, 64, 65, 1000, 4096, 5000, 6000, 10007, 16000, 32768, 65536, 65537, 100000, 200000, 300000, 500000,
+              1000000]:
+        parts, rest = divmod(floats(n, n), 10 * n)
+        assert rest == 0 and 1 <= parts <= min(64, -(-n // 64))
+        assert parts == 1 or 40 * n * parts <= 64 << 20, (n, parts)
+        blocks = -(-n // 256)
+        if n >= 4000 and 40 * n * -(-512 // blocks) <= 64 << 20:
+            assert parts * blocks >= 512, (n, parts)
+    # two instances: the first one's particles count
+    assert 32 * 10 * 100 <= floats(100, 1000000) <= 64 * 10 * 100
+    assert floats(1000000, 100) == 10 * 1000000
