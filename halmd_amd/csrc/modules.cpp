@@ -1639,6 +1639,7 @@ void verlet::integrate_kernel(double const* scale, andersen_step const* bath) {
 void verlet::integrate() { integrate_kernel(nullptr); }
 
 void verlet::finalize() {
+    p.settle_thermostat();   // another integrator's: with the force of this step, before this kick
     // (a coupled instance's force depends on the others' positions: its kick
     // must use them now, before they move again)
     if (defer_finalize && !p.coupled()) {

@@ -132,7 +132,8 @@ public:
     // settles it first.  0 = none pending.
     float pending_half_dt = 0;
     // the work that a thermostat still owes the velocities (empty: none); done
-    // by settle_velocity, or taken over by that thermostat's next half step
+    // by settle_velocity, or taken over by that thermostat's next half step.
+    // Never owed together with a kick: whoever leaves either settles first
     std::function<void()> owed_thermostat;
     void settle_velocity();
     void settle_thermostat();

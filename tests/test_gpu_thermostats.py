@@ -3,7 +3,7 @@
 import numpy as np
 import pytest
 
-from halmd_amd import workloads
+from halmd_amd import mdsim, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +45,32 @@ def test_reading_between_steps_leaves_the_trajectory(integrator, n):
             assert np.max(np.abs(a.particle.ordered(name) - b.particle.ordered(name))) < 1e-6, name
         assert np.allclose(a.integrator.position, b.integrator.position, rtol=1e-6, atol=1e-12)
         assert np.allclose(a.integrator.velocity, b.integrator.velocity, rtol=1e-6, atol=1e-9)
+
+
+def _assert_same(integrator, a, b):
+    for name in ("position", "velocity", "image"):
+        x, y = a.particle.ordered(name), b.particle.ordered(name)
+        if integrator == "verlet_nvt_andersen":
+            assert np.array_equal(x, y), name
+        else:
+            assert np.max(np.abs(x - y)) < 1e-6, name   # (as above)
+
+
+@pytest.mark.parametrize("thermostat_first", [True, False])
+@pytest.mark.parametrize("integrator", sorted(OPTIONS))
+def test_second_integrator_on_the_particle(integrator, thermostat_first):
+    # every half kick arrives, whichever integrator owes it
+    runs = []
+    for read in (False, True):
+        w = _system(integrator, 1001)
+        other = mdsim.integrators.verlet(box=w.box, particle=w.particle, timestep=0.002)
+        order = [w.integrator, other] if thermostat_first else [other, w.integrator]
+        for _ in range(8):
+            for g in order:
+                g.integrate()
+            for g in order:
+                g.finalize()
+                if read:
+                    w.particle.data["velocity"]
+        runs.append(w)
+    _assert_same(integrator, *runs)
