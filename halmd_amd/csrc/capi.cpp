@@ -62,7 +62,7 @@ kernel_timer& timer_of(void* h, char const* module) {
     if (m == "integrate" || m == "finalize") {
         auto* v = dynamic_cast<verlet*>(reinterpret_cast<integrator*>(h));
         if (!v) throw halmd::error(HALMD_ERR_INVALID_ARGUMENT, "not a Verlet integrator");
-        return m == "integrate" ? v->timer_integrate : v->timer_finalize;
+        return m == "integrate" ? v->timer_integrate : *v->timer_finalize;
     }
     if (m == "sort") return reinterpret_cast<hilbert*>(h)->timer;
     if (m == "density_mode") return reinterpret_cast<density_mode*>(h)->timer;

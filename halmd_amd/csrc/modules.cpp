@@ -1654,9 +1654,9 @@ void verlet::finalize() {
         }
     } else {
         p.update_force();
-        timer_finalize.start(p.stream);
+        timer_finalize->start(p.stream);
         launch_verlet_finalize(p.vel, p.force, p.n, ip.half_dt, p.stream);
-        timer_finalize.stop(p.stream);
+        timer_finalize->stop(p.stream);
     }
     p.velocities_changed();
 }
@@ -1744,9 +1744,9 @@ void verlet_nvt_hoover::integrate() {
 void verlet_nvt_hoover::finalize() {
     p.update_force();
     p.settle_velocity();
-    timer_finalize.start(p.stream);
+    timer_finalize->start(p.stream);
     launch_finalize_mv2(p.vel, p.force, p.n, ip.half_dt, ch->partials, p.stream);
-    timer_finalize.stop(p.stream);
+    timer_finalize->stop(p.stream);
     p.velocities_changed();
     ch->owed = true;
     p.owed_thermostat = [c = ch, &p = p] {
@@ -1787,10 +1787,12 @@ void verlet_nvt_andersen::finalize() {
     p.velocities_changed();
     last->t = {nullptr, ip.half_dt, float(rate * dt), float(std::sqrt(temperature)), seed, step++};
     last->owed = true;
-    p.owed_thermostat = [o = last, &p = p] {
+    p.owed_thermostat = [o = last, timer = timer_finalize, &p = p] {
         o->owed = false;
         o->t.id = p.id;
+        timer->start(p.stream);
         launch_andersen_finalize(p.vel, p.force, p.n, o->t, p.stream);
+        timer->stop(p.stream);
     };
 }
 

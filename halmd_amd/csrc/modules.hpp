@@ -530,7 +530,9 @@ public:
     double timestep() const override { return dt; }
     void integrate() override;
     void finalize() override;
-    kernel_timer timer_integrate, timer_finalize;
+    kernel_timer timer_integrate;
+    // (shared with the work that the particles may still owe a replaced integrator)
+    std::shared_ptr<kernel_timer> timer_finalize = std::make_shared<kernel_timer>();
     // leave the finalize kick pending for the next integrate kernel (plain
     // NVE Verlet; the thermostats need the kicked velocities at once)
     bool defer_finalize = true;

@@ -577,7 +577,11 @@ HALMD_API int halmd_server_job_release(halmd_server* s, uint64_t id);
 /* ---- profiling: per-module kernel timers (HIP events on the stream) ------ */
 /* module: "force", "neighbour", "binning", "integrate", "finalize", "sort",
  * "density_mode"; handle: the module's handle (force, neighbour, binning,
- * integrator, integrator, sort, density_mode); max_launches = 0 disables */
+ * integrator, integrator, sort, density_mode); max_launches = 0 disables.
+ * A finalize that the next integrate takes over (the kick of verlet, the
+ * collisions of verlet_nvt_andersen) is part of "integrate", or of "force"
+ * where the force kernel integrates; "finalize" counts the ones launched by
+ * themselves, as when the velocities are read in between. */
 HALMD_API int halmd_profile_enable(void* handle, const char* module, size_t max_launches);
 HALMD_API int halmd_profile_collect(void* handle, const char* module, double* total_ms, uint64_t* launches);
 

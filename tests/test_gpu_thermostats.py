@@ -1,9 +1,11 @@
 """What a thermostat leaves to the next step is done in time for every reader."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
-from halmd_amd import mdsim, workloads
+from halmd_amd import _lib, mdsim, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -74,3 +76,27 @@ def test_second_integrator_on_the_particle(integrator, thermostat_first):
                     w.particle.data["velocity"]
         runs.append(w)
     _assert_same(integrator, *runs)
+
+
+def test_profile_counts_andersen_collisions():
+    # each step's collisions are launched by "integrate" (with the next step)
+    # or by "finalize" (when the velocities are read first)
+    w = _system("verlet_nvt_andersen", 1001)
+
+    def launches(module):
+        ms, n = ctypes.c_double(), ctypes.c_uint64()
+        _lib.call("halmd_profile_collect", w.integrator.handle, module, ctypes.byref(ms), ctypes.byref(n))
+        assert (ms.value > 0) == (n.value > 0)
+        return n.value
+
+    w.sampler.run(1)   # (the first step's half is made by the force kernel)
+    for module in (b"integrate", b"finalize"):
+        _lib.call("halmd_profile_enable", w.integrator.handle, module, 100)
+    w.sampler.run(7)
+    assert (launches(b"integrate"), launches(b"finalize")) == (7, 0)
+    w.particle.data["velocity"]
+    assert (launches(b"integrate"), launches(b"finalize")) == (0, 1)
+    for _ in range(5):
+        w.sampler.run(1)
+        w.particle.data["velocity"]
+    assert (launches(b"integrate"), launches(b"finalize")) == (5, 5)
