@@ -464,9 +464,13 @@ struct build_stage {
 };
 template <>
 struct build_stage<0> {};
-// a workgroup's LDS, and what the static tables take of it
-constexpr size_t BUILD_LDS_MAX = 64 << 10, BUILD_TABLES = sizeof(seg_stage) + MAX_TYPES * MAX_TYPES * 4 + 512;
-constexpr size_t ENS_BUILD_TABLES = BUILD_TABLES + SEG_NR * SEG_BOUND * 4;
+// the most LDS that a workgroup of the list build takes (of 160 KB): the
+// largest union of records of the given size, cell bounds, tables and masks
+constexpr size_t build_lds_max(size_t record, size_t masks) {
+    return (SEG_MAX_RECORDS + 4) * record + SEG_NR * SEG_BOUND * 4 + sizeof(seg_stage) + MAX_TYPES * MAX_TYPES * 4 +
+           masks + 512;
+}
+constexpr size_t BUILD_LDS = 160 << 10;
 
 template <bool MULTI, bool ISO, bool FOLD, unsigned SPLIT>
 __device__ __forceinline__ void staged_build_segment(
@@ -1469,19 +1473,22 @@ __global__ __launch_bounds__(256) void ens_copyback_flagged_kernel(
     }
 }
 
-// the staged list build over the flagged segments
-constexpr unsigned ENS_BUILD_SPLIT = 4;   // 256 particles a pass: a segment's, most often
-template <bool MULTI, unsigned SPLIT>
-__global__ __launch_bounds__(SPLIT ? SPLIT * SPLIT_WAVES * WAVE : SEG_THREADS_MAX) void ens_build_flagged_kernel(
+// The staged list build over the flagged segments, 256 particles a pass: most
+// often a whole segment, whatever the workgroup size of the force kernels.
+// With a group for each of their waves (2, 1) it is slower: 52, 91 us (128, 64
+// threads) against 37, 63 for the 64-system ensemble.
+constexpr unsigned ENS_BUILD_SPLIT = 4, ENS_BUILD_THREADS = ENS_BUILD_SPLIT * SPLIT_WAVES * WAVE;
+static_assert(build_lds_max(sizeof(uint2), sizeof(build_stage<ENS_BUILD_SPLIT>)) <= BUILD_LDS, "");
+template <bool MULTI>
+__global__ __launch_bounds__(ENS_BUILD_THREADS) void ens_build_flagged_kernel(
     uint4 const* __restrict__ posq, uint32_t const* __restrict__ offsets, ens_desc const* __restrict__ descs,
-    uint32_t* skip, ens_work w, uint16_t* __restrict__ list, uint32_t* __restrict__ count,
-    uint32_t* __restrict__ stats)
+    uint32_t* skip, ens_work w, uint16_t* __restrict__ list, uint32_t* __restrict__ count)
 {
     extern __shared__ uint4 s_rec[];
     __shared__ seg_stage st;
     __shared__ unsigned s_bound[SEG_NR * SEG_BOUND];
     __shared__ uint32_t s_rr[MAX_TYPES * MAX_TYPES];
-    __shared__ build_stage<SPLIT> sh;
+    __shared__ build_stage<ENS_BUILD_SPLIT> sh;
     __shared__ uint32_t s_skip;
     unsigned const nl = w.head[0];
     uint32_t const total = w.lseg[nl];
@@ -1495,7 +1502,7 @@ __global__ __launch_bounds__(SPLIT ? SPLIT * SPLIT_WAVES * WAVE : SEG_THREADS_MA
         bool const skipped = s_skip != 0;
         if (!skipped) {
             ens_desc const& d = descs[s];
-            staged_build_segment<MULTI, true, false, SPLIT>(
+            staged_build_segment<MULTI, true, false, ENS_BUILD_SPLIT>(
                 posq + d.base, offsets + d.cell_base, d.sp, g - w.lseg[k], d.np, d.cap, list + d.list_off,
                 count + d.base, nullptr, s_rec, st, s_bound, s_rr, SEG_BOUND, &skip[s], sh);
         }
@@ -1595,10 +1602,8 @@ void launch_build_neighbours_staged(uint4 const* posq, unsigned n, uint32_t cons
     // second pass over one group's waves costs more than the split gains: 44
     // against 58 us at N = 64,000 with 93 a segment, 61 against 79 us for a slab
     // of 100,003 with 99)
-    auto const fits = [&](size_t stage) { return lds + stage + BUILD_TABLES <= BUILD_LDS_MAX; };
-    unsigned groups = n >= BUILD_SPLIT_BELOW ? 0 : div_up(n, sp.nseg) <= WAVE ? 1 : 2;
-    if (groups == 2 && !fits(sizeof(build_stage<2>))) groups = 0;
-    if (groups == 1 && !fits(sizeof(build_stage<1>))) groups = 0;
+    unsigned const groups = n >= BUILD_SPLIT_BELOW ? 0 : div_up(n, sp.nseg) <= WAVE ? 1 : 2;
+    static_assert(build_lds_max(sizeof(uint4), sizeof(build_stage<2>)) <= BUILD_LDS, "");
     bool const fold = p.ntype == 1 && p.iso && std::min({sp.grid.ncell[0], sp.grid.ncell[1], sp.grid.ncell[2]}) >= 5;
     auto const go = [&](auto kernel, unsigned threads) {
         kernel<<<grid, threads, lds, s>>>(posq, offset, sp, p, cap, list, count, stats);
@@ -1734,18 +1739,11 @@ void launch_ens_rebuild_device(ens_rebuild_args const& a, hipStream_t s) {
     if (a.lds_records) {
         // cubic boxes: packed records, and 4 records of slack for the scan's last group
         size_t const lds = (size_t(a.lds_records) + 4) * sizeof(uint2);
-        auto const go = [&](auto kernel, unsigned threads) {
-            kernel<<<ENS_WORK_GRID, threads, lds, s>>>(a.posq, a.offsets, a.descs, a.skip, a.w, a.list, a.count,
-                                                       a.stats);
+        auto const go = [&](auto kernel) {
+            kernel<<<ENS_WORK_GRID, ENS_BUILD_THREADS, lds, s>>>(a.posq, a.offsets, a.descs, a.skip, a.w, a.list,
+                                                                 a.count);
         };
-        constexpr unsigned T = ENS_BUILD_SPLIT * SPLIT_WAVES * WAVE;
-        bool const split = lds + sizeof(build_stage<ENS_BUILD_SPLIT>) + ENS_BUILD_TABLES <= BUILD_LDS_MAX;
-        if (a.multi)
-            split ? go(ens_build_flagged_kernel<true, ENS_BUILD_SPLIT>, T)
-                  : go(ens_build_flagged_kernel<true, 0>, SEG_THREADS_MAX);
-        else
-            split ? go(ens_build_flagged_kernel<false, ENS_BUILD_SPLIT>, T)
-                  : go(ens_build_flagged_kernel<false, 0>, SEG_THREADS_MAX);
+        a.multi ? go(ens_build_flagged_kernel<true>) : go(ens_build_flagged_kernel<false>);
         HIP_CHECK(hipGetLastError());
     }
     if (a.small_max_n) {

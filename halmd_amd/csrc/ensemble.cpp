@@ -779,7 +779,7 @@ void ensemble::enqueue_stretch(unsigned steps, unsigned build_lds, bool multi, u
         HIP_CHECK(hipStreamWaitEvent(rebuild_stream_, decided_, 0));
         ens_rebuild_args const a{pos_, vel_, image_, id_, posq_, r0_, pos_t_, vel_t_, image_t_, id_t_, posq_t_,
                                  offsets_, offsets_t_, keys_, vals_, cnt27_, base27_, bsum_, descs_, w, skip_,
-                                 threads_, build_lds, multi, small_max, list_, count_, stats_};
+                                 build_lds, multi, small_max, list_, count_, stats_};
         launch_ens_rebuild_device(a, rebuild_stream_);
         HIP_CHECK(hipEventRecord(rebuilt_, rebuild_stream_));
     }

@@ -552,7 +552,7 @@ struct ens_rebuild_args {
     ens_desc const* descs;
     ens_work w;
     uint32_t* skip;
-    unsigned threads, lds_records;   // list build (lds_records 0: no cell systems)
+    unsigned lds_records;            // list build (0: no cell systems)
     bool multi;
     unsigned small_max_n;            // 0: no all-pairs systems
     uint16_t* list;

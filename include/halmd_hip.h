@@ -518,8 +518,9 @@ HALMD_API int halmd_ensemble_recoveries(const halmd_ensemble* e, uint64_t* count
  * lists from the occupancy, from_binning.cpp:96-119) */
 HALMD_API int halmd_ensemble_set_list_capacity(halmd_ensemble* e, unsigned system, unsigned capacity);
 /* cell segments of the list build and force kernels: about `target` particles
- * per segment, `threads` per workgroup (a multiple of 64, at most 256); before
- * the first commit.  No counterpart in the reference (its launch shapes are
+ * per segment, `threads` per workgroup (a multiple of 64, at most 256) of the
+ * force kernels and of the list builds that the host decides (those decided on
+ * the device take 256 particles a pass); before the first commit.  No counterpart in the reference (its launch shapes are
  * fixed, halmd/mdsim/gpu/neighbours/from_binning.cpp:96-119); for tuners. */
 HALMD_API int halmd_ensemble_set_segments(halmd_ensemble* e, double target, unsigned threads);
 

@@ -3,7 +3,8 @@ import numpy as np
 import pytest
 from forcecheck import force_errors
 
-from halmd_amd import workloads
+from halmd_amd import mdsim, workloads
+from halmd_amd.ensemble import ensemble
 
 pytestmark = pytest.mark.gpu
 
@@ -257,6 +258,31 @@ def test_segment_shapes_change_only_the_rounding():
     ref.step(130)
     e.step(130)
     _same_trajectories(e, ref, len(SPECS))
+
+
+@pytest.mark.parametrize("threads", [64, 256])
+def test_dense_system_in_the_ensemble(threads):
+    # one system whose cells stage over 3000 records: the device's rebuilds of
+    # the others and of its own give the lists of the single-system path
+    n, steps = 20000, 60
+    L, r0, v0, _ = workloads.system_inputs(n, 0.9, 1.4, seed=3)
+    dense = (0, 1.0, 1.0, 3.5, 1.0, 1.0)   # Lennard-Jones cut at 3.5
+    e = ensemble()
+    e.set_segments(200, threads)
+    for sp in SPECS[:2]:
+        Ls, r, v, _ = workloads.system_inputs(sp["n"], sp["density"], sp["temperature"], sp["seed"])
+        e.add(r, v, Ls[0], potential=sp["potential"], timestep=DT)
+    e.add(r0, v0, L[0], potential=dense, timestep=DT)
+    e.commit()
+    e.step(steps)
+    assert e.rebuilds(2) >= 3 and e.recoveries == 0
+    for k, sp in enumerate(SPECS[:2]):
+        assert np.array_equal(e.state(k)[0], _alone(sp, steps)[0]), k
+    pot = mdsim.potentials.pair.lennard_jones(epsilon=1.0, sigma=1.0).truncate("shifted", cutoff=3.5)
+    w = workloads.fluid(n, 0.9, 1.4, pot, seed=3, timestep=DT)
+    w.sampler.run(steps)
+    for name, x in zip(("position", "velocity", "image"), e.state(2)):
+        assert np.array_equal(w.particle.ordered(name), x), name
 
 
 def test_ensemble_autotuner_returns_a_measured_choice():
