@@ -294,8 +294,8 @@ __device__ __forceinline__ void raise_to(uint32_t* word, uint32_t v) {
     if (v > __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(word, v);
 }
 
-// the pair of stats words that this workgroup raises
-__device__ __forceinline__ uint32_t* stat_pair(uint32_t* stats) {
+// the stats words that this workgroup raises
+__device__ __forceinline__ uint32_t* stat_words(uint32_t* stats) {
     return stats + blockIdx.x % STAT_SLOTS * STAT_STRIDE;
 }
 
@@ -446,16 +446,17 @@ __device__ __forceinline__ void each_hit(uint32_t m, unsigned entry0, F&& f) {
 // shared by the single-system kernel and the ensemble kernel.  The union is
 // staged as packed 16-bit records in a cubic box (8 bytes per record of the
 // dynamic LDS), else as full records (16 bytes).  stats (optional): stats[0]
-// receives the largest count, stats[1] the staging size U + 1.
+// receives the largest count, stats[1] the staging size U + 1; fullest
+// (optional) the particles of the fullest segment.
 //
 // SPLIT = 0: one lane per particle, its nine candidate rows in turn.
 // SPLIT > 0 (a workgroup of SPLIT times three waves): three waves take 64
 // particles together, one z-plane of candidate rows each.  They keep the hit
 // masks of their rows in LDS, and append them after those of the planes below,
 // whose counts the others have left there.  The tests of a lane are one chain
-// of dependent LDS reads, 47 us long at 0.84 particles per sigma^3 however few
-// particles there are; where waves are few, thirds of it side by side are
-// faster (27 us at N = 4000 and 16,000, 46 against 57 us at N = 64,000).
+// of dependent LDS reads, 50 us long at 0.84 particles per sigma^3 however few
+// particles there are; thirds of it side by side take 30 us at N = 4000 and
+// 16,000 (build_split: when).
 constexpr unsigned SPLIT_WAVES = 3, SPLIT_MASKS = 9;   // masks a lane keeps; a later one is formed again
 template <unsigned SPLIT>
 struct build_stage {
@@ -477,7 +478,7 @@ __device__ __forceinline__ void staged_build_segment(
     uint4 const* __restrict__ posq, uint32_t const* __restrict__ off, seg_params const& sp, unsigned seg,
     neighbour_params const& p, unsigned cap, uint16_t* __restrict__ list, uint32_t* __restrict__ count,
     uint32_t* __restrict__ stats, uint4* s_lds, seg_stage& st, unsigned* s_bound, uint32_t* s_rr,
-    unsigned bstride, uint32_t* overflow, build_stage<SPLIT>& sh)
+    unsigned bstride, uint32_t* overflow, build_stage<SPLIT>& sh, uint32_t* fullest = nullptr)
 {
     static_assert(!(FOLD && (MULTI || !ISO)), "");
     using rec_t = typename std::conditional<ISO, uint2, uint4>::type;
@@ -486,6 +487,7 @@ __device__ __forceinline__ void staged_build_segment(
         s_rr[threadIdx.x] = ISO ? p.rr16[threadIdx.x] : __float_as_uint(p.rr_cut_skin[threadIdx.x]);
     unsigned const U = stage_union(sp, seg, off, posq, s_rec, st, s_bound, bstride, [] { return false; });
     if (stats && threadIdx.x == 0) raise_to(&stats[1], U + 1);
+    if (fullest && threadIdx.x == 0) raise_to(fullest, st.own_pre[st.q.h]);
     if (U + 1 > sp.lds_cap) {   // uniform: the caller enlarges the staging and rebuilds
         if (overflow && threadIdx.x == 0) atomicOr(overflow, ENS_SKIP_OVERFLOW);
         return;
@@ -624,8 +626,9 @@ __global__ __launch_bounds__(SPLIT ? SPLIT * SPLIT_WAVES * WAVE : SEG_THREADS_MA
     // (3 (R + 2) rows of S + 3 words), sized to the segment shape
     unsigned* const s_bound = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(s_rec) +
                                                           size_t(sp.lds_cap) * (ISO ? sizeof(uint2) : sizeof(uint4)));
-    staged_build_segment<MULTI, ISO, FOLD, SPLIT>(posq, off, sp, seg, p, cap, list, count, stat_pair(stats), s_rec, st,
-                                                 s_bound, s_rr, sp.S + 3, nullptr, sh);
+    uint32_t* const words = stat_words(stats);
+    staged_build_segment<MULTI, ISO, FOLD, SPLIT>(posq, off, sp, seg, p, cap, list, count, words, s_rec, st, s_bound,
+                                                 s_rr, sp.S + 3, nullptr, sh, words + 2);
 }
 
 // --- cell segments with x sub-bins: per-particle candidate windows ---------
@@ -798,9 +801,8 @@ __global__ __launch_bounds__(SEG_THREADS_MAX) void build_windowed_kernel(
 
     unsigned const seg = seg_of_block(sp, blockIdx.x);
     if (seg >= sp.nseg) return;   // the whole workgroup
-    windowed_build_segment<MULTI>(posq, off, soff, sp, seg, p, cap, list, count, stat_pair(stats), s_rec, st, s_bound,
-                                  s_rr,
-                                  s_yz);
+    windowed_build_segment<MULTI>(posq, off, soff, sp, seg, p, cap, list, count, stat_words(stats), s_rec, st,
+                                  s_bound, s_rr, s_yz);
 }
 
 // --- ensembles: rebuild of a listed subset of systems --------------------
@@ -1578,8 +1580,8 @@ void launch_build_neighbours(uint4 const* posq, unsigned n, uint32_t const* offs
 
 namespace halmd {
 
-void launch_build_neighbours_staged(uint4 const* posq, unsigned n, uint32_t const* offset, seg_params const& sp,
-                                    neighbour_params const& p, unsigned cap, uint16_t* list, uint32_t* count,
+void launch_build_neighbours_staged(uint4 const* posq, unsigned n, unsigned own, uint32_t const* offset,
+                                    seg_params const& sp, neighbour_params const& p, unsigned cap, uint16_t* list, uint32_t* count,
                                     uint32_t* stats, hipStream_t s, uint32_t const* sub_offset) {
     if (!sp.nseg) return;
     unsigned const grid = SEG_XCD * sp.chunk;
@@ -1598,20 +1600,15 @@ void launch_build_neighbours_staged(uint4 const* posq, unsigned n, uint32_t cons
     }
     size_t const bounds = size_t(3) * (sp.R + 2) * (sp.S + 3) * sizeof(unsigned);
     size_t const lds = size_t(sp.lds_cap) * (p.iso ? sizeof(uint2) : sizeof(uint4)) + bounds;
-    // groups of three waves: two where a segment holds more than 64 particles (a
-    // second pass over one group's waves costs more than the split gains: 44
-    // against 58 us at N = 64,000 with 93 a segment, 61 against 79 us for a slab
-    // of 100,003 with 99)
-    unsigned const groups = n >= BUILD_SPLIT_BELOW ? 0 : div_up(n, sp.nseg) <= WAVE ? 1 : 2;
+    bool const split = build_split(n, own);
     static_assert(build_lds_max(sizeof(uint4), sizeof(build_stage<2>)) <= BUILD_LDS, "");
     bool const fold = p.ntype == 1 && p.iso && std::min({sp.grid.ncell[0], sp.grid.ncell[1], sp.grid.ncell[2]}) >= 5;
     auto const go = [&](auto kernel, unsigned threads) {
         kernel<<<grid, threads, lds, s>>>(posq, offset, sp, p, cap, list, count, stats);
     };
 #define HALMD_BUILD_STAGED(...)                                                                                       \
-    (groups == 2   ? go(build_staged_kernel<__VA_ARGS__, 2>, 2 * SPLIT_WAVES * WAVE)                                  \
-     : groups == 1 ? go(build_staged_kernel<__VA_ARGS__, 1>, SPLIT_WAVES * WAVE)                                      \
-                   : go(build_staged_kernel<__VA_ARGS__, 0>, sp.threads))
+    (split ? go(build_staged_kernel<__VA_ARGS__, 2>, 2 * SPLIT_WAVES * WAVE)                                          \
+           : go(build_staged_kernel<__VA_ARGS__, 0>, sp.threads))
     if (p.ntype > 1) {
         if (p.iso) HALMD_BUILD_STAGED(true, true, false);
         else HALMD_BUILD_STAGED(true, false, false);

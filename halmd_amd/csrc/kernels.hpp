@@ -234,18 +234,30 @@ __host__ __device__ inline size_t list16_index(size_t i, size_t k, size_t cap) {
            k % NB16_GROUP;
 }
 constexpr unsigned STAT_SLOTS = 64, STAT_STRIDE = 32;   // (128 bytes apart)
-// Single systems below BUILD_SPLIT_BELOW particles build their lists by three
-// waves per 64 particles: 27 against 48 us at N = 4000, 31 against 54 at 32,000,
-// 44 against 65 at 64,000, 61 against 69 for a slab of 100,003; 73 against 70 at
-// 108,000, 210 against 146 us at N = 524,288.
-constexpr unsigned BUILD_SPLIT_BELOW = 104 * 1024;
+// The list build of a single system by two groups of three waves, each with 64
+// particles a pass (own: the particles of the fullest segment), or by one lane
+// per particle.
+//  - Faster while every segment takes one pass: 45 against 58 us at N = 72,000
+//    (LJ, fullest segment 99), 65 against 79 at 90,000 (two species, 119), 51
+//    against 60 for a slab of 100,000 (119); with segments of 3 x 2 cells also 108
+//    against 131 us at 262,143 and 345 against 386 us at 2^20 (slab).
+//  - Slower once some take a second pass: 67 against 64 us at N = 86,000 (LJ, 175
+//    of 768 segments), 117 against 97 at 106,000 (two species, 177 of 960), 78
+//    against 67 at 100,000 (dilute LJ, 133 of 918).  One to three such segments
+//    go either way (64 against 91, 66 against 57 us).
+//  - Where a segment leaves most lanes idle, the system has to be small: with 19
+//    in each, 30 against 51 us at N = 16,000, 135 against 127 at 130,000, 973 against
+//    741 us at 2^20; with 37, 83 against 86 us at 130,000, 143 against 137 at 262,143.
+// (One group is never faster than two.  Three and four, which save the second
+// pass, are within 8% of one lane per particle from 80,000 on.)
+inline bool build_split(unsigned n, unsigned own) { return own <= 2 * WAVE && (own > 48 || n < (1u << 17)); }
 //
 // With sub_offset (the offsets of the (cell, x sub-bin) order the particles
 // are in, ncells SUB_BINS + 1 entries; cubic box, nx >= 4) each lane scans
 // only the candidate windows its position allows (same lists); the dynamic
 // LDS is then windowed_build_lds() bytes.
-void launch_build_neighbours_staged(uint4 const* posq, unsigned n, uint32_t const* offset, seg_params const& sp,
-                                    neighbour_params const& p, unsigned cap, uint16_t* list, uint32_t* count,
+void launch_build_neighbours_staged(uint4 const* posq, unsigned n, unsigned own, uint32_t const* offset,
+                                    seg_params const& sp, neighbour_params const& p, unsigned cap, uint16_t* list, uint32_t* count,
                                     uint32_t* stats, hipStream_t s, uint32_t const* sub_offset = nullptr);
 constexpr unsigned WIN_MAX = 10;   // candidate windows per lane: 9 rows, the own row split
 inline size_t windowed_build_lds(seg_params const& sp) {

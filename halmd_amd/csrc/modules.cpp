@@ -1170,6 +1170,7 @@ void neighbour::plan_segments(unsigned S, unsigned R) {
     sp.nsy = unsigned(div_up(ny, sp.R));
     sp.nseg = sp.nsx * sp.nsy * bin->grid.ncell[2];
     sp.chunk = unsigned(div_up(sp.nseg, SEG_XCD));
+    fullest = 0;
 }
 
 void neighbour::require_current() {
@@ -1255,18 +1256,23 @@ void neighbour::update(double displacement_bound) {
     while (true) {
         timer.start(s);
         bool const win = windows && windowed_build_lds(sp) <= lds_bytes;
-        launch_build_neighbours_staged(p.posq, p.n, bin->order_offset, sp, params, cap, list16, count, d_maxcount, s,
-                                       win ? bin->order_sub_offset.get() : nullptr);
+        // (a first build goes by the mean, with a margin for the fullest segment)
+        unsigned const own = fullest ? fullest : unsigned(1.15 * mean_occupancy() * sp.S * sp.R);
+        launch_build_neighbours_staged(p.posq, p.n, own, bin->order_offset, sp, params, cap, list16, count,
+                                       d_maxcount, s, win ? bin->order_sub_offset.get() : nullptr);
         timer.stop(s);
-        // the largest count, the largest union and the merge check of the
-        // binning (0 when it sorted), polled as they are stored, and reset
-        mailbox_sources const src{{d_maxcount.get(), d_maxcount.get() + 1, bin->merge_check_word(), nullptr},
-                                  {STAT_SLOTS, STAT_SLOTS, 1, 0},
-                                  {STAT_STRIDE, STAT_STRIDE, 1, 0}};
-        uint32_t got[3];
-        build_box.wait(build_box.post(src, 3, s), 3, got, s);
+        // the largest count, the largest union, the merge check of the binning
+        // (0 when it sorted) and the fullest segment (0 from the windowed
+        // build), polled as they are stored, and reset
+        uint32_t* const st = d_maxcount.get();
+        mailbox_sources const src{{st, st + 1, bin->merge_check_word(), st + 2},
+                                  {STAT_SLOTS, STAT_SLOTS, 1, STAT_SLOTS},
+                                  {STAT_STRIDE, STAT_STRIDE, 1, STAT_STRIDE}};
+        uint32_t got[4];
+        build_box.wait(build_box.post(src, 4, s), 4, got, s);
         bin->merge_checked(got[2]);
         unsigned const m = got[0], u = got[1];
+        fullest = got[3];
         if (u > sp.lds_cap) {
             // a union outgrew the staging: enlarge it, else narrow the segments
             if (u + u / 8 <= lds_limit) {

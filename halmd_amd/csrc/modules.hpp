@@ -383,6 +383,7 @@ public:
     // cell-segment lists (this module keeps the particles in cell order)
     bool staged = false;
     seg_params sp{}, sp_force{};      // build staging / force staging (lds_cap = largest union)
+    unsigned fullest = 0;             // particles of the last build's fullest segment (0: none of this shape)
     size_t lds_limit = 0;             // records of dynamic LDS a build workgroup may use
     size_t lds_bytes = 0;             // dynamic LDS bytes a build workgroup may use
     bool windows = false;             // windowed list build over the (cell, x sub-bin) order

@@ -36,6 +36,40 @@ def test_shape_leaves_lists(oracle, kind, n):
         assert np.array_equal(entries[valid], lists[valid])
 
 
+def _fullest(w):
+    """Particles of the fullest segment."""
+    nc, (S, R, _) = np.asarray(w.neighbour.binning.ncell, dtype=np.uint64), w.neighbour.segments
+    c = (w.particle.data["position_fixed"].astype(np.uint64) * nc) >> np.uint64(32)
+    return np.unique(np.stack([c[:, 0] // np.uint64(S), c[:, 1] // np.uint64(R), c[:, 2]]), axis=1,
+                     return_counts=True)[1].max()
+
+
+# (2^17: from here on segments of few particles are built by one lane each)
+@pytest.mark.parametrize("n,shapes", [(4001, [(3, 1, 256), (2, 2, 256), (3, 2, 128)]),
+                                      (32000, [(2, 2, 256), (5, 1, 256), (3, 2, 256)]),
+                                      ((1 << 17) - 1, [(2, 1, 256), (3, 1, 256)]), (1 << 17, [(2, 1, 256), (3, 1, 256)])])
+def test_lists_either_side_of_one_pass(oracle, n, shapes):
+    # 128 particles: a pass of the list build by three waves; the fullest segment
+    # of one build chooses the next one's kernel
+    w = _system("lj", n, 0.15)
+    w.neighbour.update()
+    counts, entries = w.neighbour.lists()
+    u, species = w.particle.data["position_fixed"], w.particle.data["species"]
+    expect, lists, _ = oracle.staged_neighbour_list(u, species, w.neighbour.binning.ncell, w.length,
+                                                    w.potential.r_cut + w.skin, entries.shape[1])
+    valid = np.arange(entries.shape[1]) < expect[:, None]
+    fullest = []
+    for shape in shapes:
+        w.neighbour.set_segments(*shape)
+        fullest.append(_fullest(w))
+        for _ in range(2):
+            w.neighbour.update()
+            counts, entries = w.neighbour.lists()
+            assert np.array_equal(counts, expect)
+            assert np.array_equal(entries[valid], lists[valid])
+    assert min(fullest) <= 128 and (max(fullest) > 128 or n >= (1 << 17) - 1), fullest
+
+
 @pytest.mark.parametrize("kind,n", [("lj", 1372), ("lj", 4001), ("ka", 8788), ("lj", 262143)])
 def test_shape_leaves_trajectory(kind, n):
     runs = []
