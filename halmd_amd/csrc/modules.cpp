@@ -1087,7 +1087,7 @@ void neighbour::init(double const* rc, unsigned nt1, unsigned nt2) {
         windows = params.iso && bin->grid.ncell[0] >= 4 && ew && std::atoi(ew) != 0;
         // (pair_trunc::tune refines the width by measurement)
         unsigned S, R;
-        segment_shape(mean_occupancy(), bin->grid, segment_target(p.n), S, R);
+        default_segments(p.n, bin->grid, S, R);
         set_segments(S, R, SEG_THREADS_MAX);
     } else {
         cap = unsigned(round_up(size_t(std::ceil(nmean / occupancy)) + NB_BLOCK, NB_BLOCK));
@@ -1136,19 +1136,42 @@ void segment_shape(double occupancy, cell_grid const& g, double target, unsigned
 
 double segment_target(unsigned n) {
     if (char const* e = std::getenv("HALMD_SEG_TARGET")) return std::max(1.0, std::atof(e));
-    // The staging of a segment's union is paid per segment, so up to the 256
-    // threads of a workgroup larger is better where there are workgroups enough;
-    // below N = 160,000 there are not, and about 800 segments are best: the
-    // whole step (force, integration, its share of the list build) takes 22
-    // against 28 us with segments of 200 at N = 4000, 20 against 28 at 16,000,
-    // 22 against 26 at 64,000, 35 against 39 at 108,000, the same from 160,000.
-    // (One to two cells a segment at the least: smaller workgroups stage more
-    // than they own.)
-    if (n < FORCE_STREAMS_BELOW) return std::clamp(n / 800.0, 32.0, 200.0);
-    // Here the sums follow the shape, so an ensemble's systems of this size
-    // take the same (200 against 230: 76 against 80 us at N = 524,288, 140
-    // against 136 at N = 2^20).
+    // The staging of a segment's union is paid per segment, so larger is better
+    // up to about the 256 threads of a workgroup: a step of 4 x 3 cells against
+    // 3 x 3 takes 98 against 96 us at N = 700,000, 109 against 113 at 786,432, 134
+    // against 139 at 2^20, 496 against 520 at 4,000,000 (LJ; dilute or in a slab
+    // within 4% of each other)
     return n < 3 * FORCE_STREAMS_BELOW ? 200 : 230;
+}
+
+void default_segments(unsigned n, cell_grid const& g, unsigned& S, unsigned& R) {
+    double const occupancy = double(n) / (double(g.ncell[0]) * g.ncell[1] * g.ncell[2]);
+    unsigned most = 0;
+    if (n < FORCE_STREAMS_BELOW && !std::getenv("HALMD_SEG_TARGET")) {
+        // The most segments that run at the same time, four workgroups on each of
+        // 256 compute units: with fewer the chip is not full, with more a second
+        // round begins.  A step of 72,000 particles (two species) takes 29.6 us with
+        // 845 segments of 3 x 1 cells, 35.6 with 1183, 33.5 with 637; of 108,000
+        // 30.4 with 1024, 35.7 with 768; of 150,000 (LJ) 34.4 with 1000, 36.1 with
+        // 980, 41.5 with 1400; of 230,000 (two species) 44.0 with 1000, 52.6 with
+        // 1400, 54.8 with 700.  Near square, and of 20 to 240 particles (smaller
+        // ones stage more than they own; from 256 on a thread takes two); above 200
+        // only where the rows divide evenly (LJ at 180,000: 44.6 us with 882 of 4 x
+        // 3, 6 columns in 21 cells, 39.4 with 1029 of 3 x 3).  Where there is no such
+        // shape, the target of large systems.
+        for (unsigned r = 1; r <= std::min(SEG_RMAX, g.ncell[1] - 2); ++r)
+            for (unsigned s = 1; s <= std::min({SEG_MAX, g.ncell[0] - 2, 2 * r + 1}); ++s) {
+                double const own = occupancy * s * r;
+                if (r > 2 * s + 1 || own < 20 || own > 240) continue;
+                unsigned const nseg = unsigned(div_up(g.ncell[0], s) * div_up(g.ncell[1], r) * g.ncell[2]);
+                if (nseg > 1024 || nseg < most || (own > 200 && own * nseg > 1.11 * n)) continue;
+                if (nseg == most && (s * r > S * R || (s * r == S * R && s + r >= S + R))) continue;
+                most = nseg;
+                S = s;
+                R = r;
+            }
+    }
+    if (!most) segment_shape(occupancy, g, segment_target(n), S, R);
 }
 
 double neighbour::mean_occupancy() const { return bin ? double(p.n) / bin->ncells : 0.0; }

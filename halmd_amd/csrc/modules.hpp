@@ -346,9 +346,11 @@ class hilbert;
 // particles at the given mean cell occupancy (within the grid's limits)
 void segment_shape(double occupancy, cell_grid const& g, double target, unsigned& S, unsigned& R);
 
-// particles per segment of a system of n particles that has the chip to itself
-// (HALMD_SEG_TARGET overrides)
+// particles per segment of a large system (HALMD_SEG_TARGET overrides)
 double segment_target(unsigned n);
+
+// the segments of a system of n particles that has the chip to itself
+void default_segments(unsigned n, cell_grid const& g, unsigned& S, unsigned& R);
 
 class neighbour {
 public:

@@ -226,3 +226,34 @@ def test_pair_full_scratch_and_workgroups():
     # two instances: the first one's particles count
     assert 32 * 10 * 100 <= floats(100, 1000000) <= 64 * 10 * 100
     assert floats(1000000, 100) == 10 * 1000000
+
+
+@pytest.mark.parametrize("cells", [1.0, 2.0])
+def test_default_segments_run_at_the_same_time(cells, monkeypatch):
+    # below 2^18 particles the most segments of 20 to 240 particles, at most four
+    # for each of the 256 compute units (above 200 particles only where the rows
+    # divide evenly); cells: of a cubic box, of one twice as long
+    monkeypatch.delenv("HALMD_SEG_TARGET", raising=False)
+    plan = _lib.lib()["_ZN5halmd16default_segmentsEjRKNS_9cell_gridERjS3_"]
+    plan.restype = None
+    plan.argtypes = [ctypes.c_uint] + [ctypes.c_void_p] * 3
+    found = 0
+    for occupancy in (2.5, 9.0, 19.0, 24.0, 32.0, 55.0):
+        for n in (150, 1000, 4000, 16000, 40000, 72000, 100000, 108000, 150000, 180000, 230000, (1 << 18) - 1, 1 << 18):
+            edge = max(3, round((n / occupancy / cells) ** (1 / 3)))
+            g = np.array([edge, edge, max(3, round(edge * cells))], dtype=np.uint32)
+            S, R = ctypes.c_uint(), ctypes.c_uint()
+            plan(n, g.ctypes.data, ctypes.addressof(S), ctypes.addressof(R))
+            S, R = S.value, R.value
+            assert 1 <= S <= min(32, g[0] - 2) and 1 <= R <= min(8, g[1] - 2)
+            mean = n / float(np.prod(g))
+            nseg = lambda s, r: int(-(-int(g[0]) // s) * -(-int(g[1]) // r) * int(g[2]))
+            shapes = [(s, r) for r in range(1, min(8, int(g[1]) - 2) + 1) for s in range(1, min(32, int(g[0]) - 2) + 1)
+                      if s <= 2 * r + 1 and r <= 2 * s + 1 and 20 <= mean * s * r <= 240 and nseg(s, r) <= 1024
+                      and (mean * s * r <= 200 or mean * s * r * nseg(s, r) <= 1.11 * n)]
+            if n < 1 << 18 and shapes:
+                found += 1
+                assert nseg(S, R) == max(nseg(s, r) for s, r in shapes), (n, g, S, R)
+            elif min(g) > 8 and mean < 200:
+                assert 100 < mean * S * R < 330, (n, g, S, R)
+    assert found > 40
