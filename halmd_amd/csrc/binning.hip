@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void build_all_pairs_kernel(uint4 const* __res
     unsigned const i0 = blockIdx.x * AP_PER_GROUP;
     if (cond.slots) {
         // the whole workgroup
-        if (!displacement_aborts(displacement_word(cond.slots), cond.slots, cond.keep_bits)) return;
+        if (!displacement_aborts(cond.slots, cond.keep_bits)) return;
         if (threadIdx.x < AP_PER_GROUP && i0 + threadIdx.x < n)
             cond.r0[i0 + threadIdx.x] = cond.pos[2 * size_t(i0 + threadIdx.x)];
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(cond.rebuilt, 1u);
@@ -485,7 +485,7 @@ __device__ __forceinline__ void staged_build_segment(
     rec_t* const s_rec = reinterpret_cast<rec_t*>(s_lds);
     if (threadIdx.x < MAX_TYPES * MAX_TYPES)
         s_rr[threadIdx.x] = ISO ? p.rr16[threadIdx.x] : __float_as_uint(p.rr_cut_skin[threadIdx.x]);
-    unsigned const U = stage_union(sp, seg, off, posq, s_rec, st, s_bound, bstride, [] { return false; });
+    unsigned const U = stage_union(sp, seg, off, posq, s_rec, st, s_bound, bstride);
     if (stats && threadIdx.x == 0) raise_to(&stats[1], U + 1);
     if (fullest && threadIdx.x == 0) raise_to(fullest, st.own_pre[st.q.h]);
     if (U + 1 > sp.lds_cap) {   // uniform: the caller enlarges the staging and rebuilds
@@ -662,7 +662,7 @@ __device__ __forceinline__ void windowed_build_segment(
 {
     uint2* const s_rec = reinterpret_cast<uint2*>(s_lds);
     if (threadIdx.x < MAX_TYPES * MAX_TYPES) s_rr[threadIdx.x] = p.rr16[threadIdx.x];
-    unsigned const U = stage_union(sp, seg, off, posq, s_rec, st, s_bound, SEG_BOUND, [] { return false; });
+    unsigned const U = stage_union(sp, seg, off, posq, s_rec, st, s_bound);
     if (stats && threadIdx.x == 0) raise_to(&stats[1], U + 1);
     if (U + 1 > sp.lds_cap) return;   // uniform: the caller enlarges the staging and rebuilds
 

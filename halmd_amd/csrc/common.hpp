@@ -226,8 +226,8 @@ __device__ __forceinline__ uint32_t dpp(uint32_t other, uint32_t v) {
 }
 
 // The wave scans go up the lanes of each row of 16 (row shifts), then across
-// the rows (row broadcasts): seven VALU instructions, where shuffles through
-// LDS take six dependent LDS round trips.
+// the rows (row broadcasts): six VALU instructions, where shuffles through LDS
+// take six dependent LDS round trips.
 __device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t x) {
     x += dpp<0x111>(0u, x);        // row_shr 1
     x += dpp<0x112>(0u, x);

@@ -409,7 +409,7 @@ __device__ __forceinline__ float staged_force_segment(
         ISO && KIND == POTENTIAL_LENNARD_JONES && (TRUNC == TRUNC_SHARP || TRUNC == TRUNC_SHIFTED);
     constexpr bool P0_OUT = LJQ && !MULTI;   // 48 eps / sigma^2 applied per particle
     if (MULTI && threadIdx.x < MAX_TYPES * MAX_TYPES) s_pair[threadIdx.x] = P.pair[threadIdx.x];
-    stage_union(sp, seg, off, posq, s_rec, st, nullptr, 0u, [] { return false; });   // fits: the list build checked it
+    stage_union(sp, seg, off, posq, s_rec, st, nullptr);   // fits: the list build checked it
 
     unsigned const T = st.own_pre[st.q.h];
     unsigned const lane = threadIdx.x % WAVE;
@@ -650,7 +650,7 @@ __global__ __launch_bounds__(SEG_THREADS_MAX) void pair_force_staged_kernel(
     unsigned const seg = seg_of_block(sp, blockIdx.x);   // workgroup 0 has segment 0
     if (seg >= sp.nseg) return;   // the whole workgroup
     // the whole workgroup
-    if (displacement_aborts(displacement_word(chk.slots), chk.slots, chk.bits, chk.publish, chk.seq)) return;
+    if (displacement_aborts(chk.slots, chk.bits, chk.publish, chk.seq)) return;
     float const d2 = staged_force_segment<KIND, TRUNC, AUX, ISO, MULTI, FUSE, STREAMS>(
         posq, off, sp, seg, list, count, cap, P, force_zero, aux_weight, force, stress, stride, s_rec, st, s_pair, &F);
     if (FUSE) {

@@ -48,15 +48,11 @@ __device__ __forceinline__ void seg_own(seg_stage const& st, unsigned t, unsigne
 // decision is uniform without a barrier.  publish (optional): lane 0 of
 // workgroup 0 stores (seq << 32) | the largest word into publish[seq %
 // PUBLISH_RING], host-mapped memory, by a vector store at system scope.
-__device__ __forceinline__ unsigned displacement_word(uint32_t const* __restrict__ slots) {
-    static_assert(DISP_SLOTS == WAVE, "one displacement slot per lane");
-    return slots ? slots[(threadIdx.x % WAVE) * DISP_STRIDE] : 0u;
-}
-// (m: the displacement_word of each lane)
-__device__ __forceinline__ bool displacement_aborts(unsigned m, uint32_t const* __restrict__ slots, uint32_t bits,
+__device__ __forceinline__ bool displacement_aborts(uint32_t const* __restrict__ slots, uint32_t bits,
                                                     unsigned long long* publish = nullptr, uint32_t seq = 0) {
     if (!slots) return false;
-    m = wave_max_u32(m);
+    static_assert(DISP_SLOTS == WAVE, "one displacement slot per lane");
+    unsigned const m = wave_max_u32(slots[(threadIdx.x % WAVE) * DISP_STRIDE]);
     if (publish && blockIdx.x == 0 && threadIdx.x == 0)
         __hip_atomic_store(publish + seq % PUBLISH_RING, (static_cast<unsigned long long>(seq) << 32) | m,
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -83,11 +79,6 @@ __device__ __forceinline__ void put_rec(uint2* s, unsigned k, uint4 const r) { s
 // particles in both (h <= ny - 2, nz >= 3).  Returns the union size U; every
 // thread sees the same value.
 //
-// early() is called by every thread once st is complete (but for the staged
-// records), before the staging loads: a caller issues its own loads there, so
-// that they share the staging's memory latency.  It returns true (for the
-// whole workgroup) to leave at once; stage_union then returns ~0u.
-//
 // Bound: latency.  A workgroup's time is a chain of dependent memory round
 // trips (about 1 us each from another XCD's writes), and below some 10^5
 // particles every workgroup of the launch runs at the same time, so the chain
@@ -97,10 +88,10 @@ __device__ __forceinline__ void put_rec(uint2* s, unsigned k, uint4 const r) { s
 // division, no branch), forms the prefix sums by DPP scans and lists the
 // 64-record chunks of the rows; then the waves take the chunks in turn, four
 // loads in flight per lane.
-template <class Dst, class Early>
+template <class Rec>
 __device__ __forceinline__ unsigned stage_union(seg_params const& sp, unsigned seg, uint32_t const* __restrict__ off,
-                                                uint4 const* __restrict__ posq, Dst const& s_rec, seg_stage& st,
-                                                unsigned* bound, unsigned bstride, Early&& early) {
+                                                uint4 const* __restrict__ posq, Rec* s_rec, seg_stage& st,
+                                                unsigned* bound, unsigned bstride = SEG_BOUND) {
     unsigned const tid = threadIdx.x, lane = tid % WAVE;
     unsigned const nx = sp.grid.ncell[0], ny = sp.grid.ncell[1], nz = sp.grid.ncell[2];
     if (tid < WAVE) {
@@ -145,7 +136,6 @@ __device__ __forceinline__ unsigned stage_union(seg_params const& sp, unsigned s
     __syncthreads();
     seg_place const q = st.q;
     unsigned const nr = st.nr, U = st.base[nr];
-    if (early()) return ~0u;   // the whole workgroup
     if (bound) {
         // LDS start of cell x0 - 1 + k (periodic) of union row ur, one thread each
         unsigned const nk = q.w + 3, hh = q.h + 2;
