@@ -1581,8 +1581,8 @@ void launch_build_neighbours(uint4 const* posq, unsigned n, uint32_t const* offs
 namespace halmd {
 
 void launch_build_neighbours_staged(uint4 const* posq, unsigned n, unsigned own, uint32_t const* offset,
-                                    seg_params const& sp, neighbour_params const& p, unsigned cap, uint16_t* list, uint32_t* count,
-                                    uint32_t* stats, hipStream_t s, uint32_t const* sub_offset) {
+                                    seg_params const& sp, neighbour_params const& p, unsigned cap, uint16_t* list,
+                                    uint32_t* count, uint32_t* stats, hipStream_t s, uint32_t const* sub_offset) {
     if (!sp.nseg) return;
     unsigned const grid = SEG_XCD * sp.chunk;
     if (sub_offset) {

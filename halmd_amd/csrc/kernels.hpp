@@ -225,15 +225,17 @@ __host__ __device__ inline void seg_own_row(seg_params const& sp, seg_place cons
 // particle i (memory order) at
 // (i / 64) * 64 * cap + (k / 8) * 512 + (i % 64) * 8 + k % 8 (uint16 units; a
 // group of 8 entries is one load of a lane, and a wave's 64 groups are 1 KiB in
-// a row)
+// a row; cap a multiple of 16).  The all-pairs systems of an ensemble share the
+// array with another layout, blocks of 16 entries: their kernels read entry k of
+// a particle by lane k % 16 (ens_build_small*, ens_force_small), at
+// (i / 64) * 64 * cap + (k / 16) * 1024 + (i % 64) * 16 + k % 16.
 constexpr unsigned NB16_GROUP = 8;
-constexpr unsigned NB16_BLOCK = 16;   // (list capacities are multiples of it)
+constexpr unsigned NB16_BLOCK = 16;   // the all-pairs systems' blocks; list capacities are multiples of it
 constexpr unsigned SEG_MAX_RECORDS = 4096;   // staged union plus sentinel
 __host__ __device__ inline size_t list16_index(size_t i, size_t k, size_t cap) {
     return (i & ~size_t(WAVE - 1)) * cap + (k / NB16_GROUP) * WAVE * NB16_GROUP + (i & (WAVE - 1)) * NB16_GROUP +
            k % NB16_GROUP;
 }
-constexpr unsigned STAT_SLOTS = 64, STAT_STRIDE = 32;   // (128 bytes apart)
 // The list build of a single system by two groups of three waves, each with 64
 // particles a pass (own: the particles of the fullest segment), or by one lane
 // per particle.
@@ -251,14 +253,28 @@ constexpr unsigned STAT_SLOTS = 64, STAT_STRIDE = 32;   // (128 bytes apart)
 // (One group is never faster than two.  Three and four, which save the second
 // pass, are within 8% of one lane per particle from 80,000 on.)
 inline bool build_split(unsigned n, unsigned own) { return own <= 2 * WAVE && (own > 48 || n < (1u << 17)); }
+
+// Builds the lists of particles in cell order.  Lists are padded with the
+// slot U of a sentinel record (staged after the union, at least a cell width
+// away from every particle of the segment in y and z) to a multiple of 8
+// entries; count[i] excludes the padding and may exceed cap (the entries past
+// cap are not stored, and the caller retries with larger lists).
+// stats: STAT_SLOTS groups of words, STAT_STRIDE words apart (one word would be
+// an atomic hot spot), each raised by a share of the workgroups; the largest
+// over the groups is the result.  Word 0: largest count; 1: largest staging size
+// U + 1 (a segment whose staging exceeds sp.lds_cap builds nothing; the caller
+// retries); 2: particles of the fullest segment (not by the windowed build).
+// All are 0 before the launch: launch_post_words resets them as it reads.
 //
 // With sub_offset (the offsets of the (cell, x sub-bin) order the particles
 // are in, ncells SUB_BINS + 1 entries; cubic box, nx >= 4) each lane scans
 // only the candidate windows its position allows (same lists); the dynamic
 // LDS is then windowed_build_lds() bytes.
+constexpr unsigned STAT_SLOTS = 64, STAT_STRIDE = 32;   // (128 bytes apart)
 void launch_build_neighbours_staged(uint4 const* posq, unsigned n, unsigned own, uint32_t const* offset,
-                                    seg_params const& sp, neighbour_params const& p, unsigned cap, uint16_t* list, uint32_t* count,
-                                    uint32_t* stats, hipStream_t s, uint32_t const* sub_offset = nullptr);
+                                    seg_params const& sp, neighbour_params const& p, unsigned cap, uint16_t* list,
+                                    uint32_t* count, uint32_t* stats, hipStream_t s,
+                                    uint32_t const* sub_offset = nullptr);
 constexpr unsigned WIN_MAX = 10;   // candidate windows per lane: 9 rows, the own row split
 inline size_t windowed_build_lds(seg_params const& sp) {
     return (size_t(sp.lds_cap) + 3) * 8 + size_t(3) * (sp.R + 2) * ((sp.S + 2) * SUB_BINS + 1) * 4 +
