@@ -78,6 +78,42 @@ def test_second_integrator_on_the_particle(integrator, thermostat_first):
     _assert_same(integrator, *runs)
 
 
+def _replace_integrator(w):
+    w.replaced = w.integrator   # (kept: its chain is still owed)
+    w.integrator = mdsim.integrators.verlet(box=w.box, particle=w.particle, timestep=0.004)
+    w.core.set_integrator(w.integrator)
+
+
+def _write_positions(w):
+    r = w.particle.data["position"]
+    w.particle.data["position"] = np.roll(r, 1, axis=0)
+
+
+def _write_mass(w):
+    w.particle.data["mass"] = np.where(w.particle.data["id"] % 3 == 0, 2.0, 1.0)
+
+
+def _add_force(w):
+    soft = mdsim.potentials.pair.power_law(epsilon=0.1, sigma=1.0, index=6)
+    w.second = mdsim.forces.pair_full(box=w.box, particle=w.particle, potential=soft)
+
+
+@pytest.mark.parametrize("event", [_replace_integrator, _write_positions, _write_mass, _add_force])
+@pytest.mark.parametrize("integrator", sorted(OPTIONS))
+def test_changes_between_steps_come_after_what_is_owed(integrator, event):
+    # the same change with the velocities read before it, which has everything done
+    runs = []
+    for read in (False, True):
+        w = _system(integrator, 1001)
+        w.sampler.run(7)
+        if read:
+            w.particle.data["velocity"]
+        event(w)
+        w.sampler.run(5)
+        runs.append(w)
+    _assert_same(integrator, *runs)
+
+
 def test_profile_counts_andersen_collisions():
     # each step's collisions are launched by "integrate" (with the next step)
     # or by "finalize" (when the velocities are read first)
