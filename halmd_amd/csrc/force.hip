@@ -527,6 +527,23 @@ __device__ __forceinline__ float staged_force_segment(
         auto group_at = [&](unsigned g) { return lp[min(g, last) * WAVE]; };
         float r[NS] = {};
         if constexpr (STREAMS) {
+            // The second stream is added to the first.  That rounds twice more
+            // than one compensated sum would, which a force or the stress does not
+            // show beside the error of its terms (5e-7, 3e-7); the energy does
+            // (6.5e-8 for 6.2e-8 of it), so it joins with its compensation: the sum
+            // is r[EN] - re.
+            constexpr int EN = 3;
+            float re = 0.0f;
+            auto join = [&](int c, float f, float g) {
+                if (c != EN) {
+                    r[c] += f - g;
+                } else {
+                    float t, e;
+                    two_sum(r[c], f, t, e);
+                    r[c] = t;
+                    re = (re + g) - e;
+                }
+            };
             // one lane per particle: both streams, one after the other (one set
             // of sums in registers; both at once take 30 more, for a wave per
             // SIMD less); two lanes: the lane's own
@@ -544,13 +561,15 @@ __device__ __forceinline__ float staged_force_segment(
                     w1 = n1;
                 }
 #pragma unroll
-                for (int c = 0; c < NS; ++c) r[c] += a.f[c] - a.c[c];
+                for (int c = 0; c < NS; ++c) join(c, a.f[c], a.c[c]);
             }
             if (k > 1) {   // wave-uniform
                 int const sl = int(lane + active < WAVE ? lane + active : lane);
+                float const other = AUX ? __shfl(re, sl, WAVE) : 0.0f;
 #pragma unroll
-                for (int c = 0; c < NS; ++c) r[c] += __shfl(r[c], sl, WAVE);
+                for (int c = 0; c < NS; ++c) join(c, __shfl(r[c], sl, WAVE), c == EN ? other : 0.0f);
             }
+            if constexpr (AUX) r[EN] -= re;
         } else {
             unsigned const nblk = (n8 / NB16_GROUP + 1) / 2;   // blocks of two groups
             unsigned const b_begin = mine ? nblk * part / k : 0u;
