@@ -590,8 +590,9 @@ def main():
         # (n_nb + 1) list words of 4 B (entries + count), force (12 B)
         force_bytes = N * (24 + 4 * (n_nb + 1) + 12)
     achieved = force_bytes / (f_avg * 1e-3) / 1e9
-    kname = ("pair_force_staged_kernel<0, 1, false, true, false, %s>" % ("true" if fused else "false") if staged
-             else "pair_force_kernel<0, 1, false>")
+    # <LJ, shifted, no sums, cubic, one species, fused, one pass over the list>
+    kname = ("pair_force_staged_kernel<0, 1, false, true, false, %s, false>" % ("true" if fused else "false")
+             if staged else "pair_force_kernel<0, 1, false>")
     prof = counter_summary(kname)
     traffic = prof.get("traffic_bytes_per_launch")
     kernels = {k: {"launches": int(n), "avg_ms": (ms_ / n if n else None)} for k, (ms_, n) in kt.items()}
