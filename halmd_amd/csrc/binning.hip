@@ -327,7 +327,7 @@ __device__ __forceinline__ unsigned nb16_count(nb16_state const& s) {
 // a wave's groups share 1 KiB, so the lines are complete in L2 before they are
 // written back; but each lane's store is a request of its own to L2, and with
 // 2-byte stores the 84 million requests of a build at N = 2^20 are its bound
-// (128 channels, one request a cycle each: 0.3 ms; 350 us, 263 us packed).
+// (128 channels, one request a cycle each: 0.3 ms; 350 us, packed 276 us).
 // The split build of small systems (below) starts at any entry and stores each
 // by itself: there the appends' latency counts (42 against 50 us at N = 16,000
 // with one lane per particle).
@@ -1399,9 +1399,9 @@ __global__ __launch_bounds__(256) void ens_scatter_kernel(
 // gather by it, an identity fill and a copy of the offsets; most particles keep
 // their cell, so the writes go out as whole lines like those of a gather.  With
 // skip set every particle keeps its slot and the offsets stay.
-// A rebuild of 4000 particles takes 6 launches before and after the list build
-// in place of 12 (92 us in all against 130); the pass itself 49 us at N = 2^20,
-// as long as the gather alone.
+// A rebuild of 4000 particles takes 6 launches, the list build among them, in
+// place of 11 (92 us in all against 130); the pass itself 48 us at N = 2^20, as
+// long as the gather alone.
 __global__ __launch_bounds__(256) void merge_scatter_kernel(rearrange_arrays a, unsigned n, unsigned C,
                                                             uint32_t const* skip, uint32_t const* __restrict__ keys,
                                                             uint32_t const* __restrict__ rank,
@@ -1477,8 +1477,10 @@ __global__ __launch_bounds__(256) void ens_copyback_flagged_kernel(
 
 // The staged list build over the flagged segments, 256 particles a pass: most
 // often a whole segment, whatever the workgroup size of the force kernels.
-// With a group for each of their waves (2, 1) it is slower: 52, 91 us (128, 64
-// threads) against 37, 63 for the 64-system ensemble.
+// For an ensemble of 64 systems 36 us, 60 with one lane for each particle; a group
+// for each wave of a smaller force workgroup is slower (128 threads: 52 against
+// 35-49 us, 64: 91 against 63).  For 256 systems, which fill the chip by
+// themselves, 140 us against 131 with one lane for each, a step 0.6% longer.
 constexpr unsigned ENS_BUILD_SPLIT = 4, ENS_BUILD_THREADS = ENS_BUILD_SPLIT * SPLIT_WAVES * WAVE;
 static_assert(build_lds_max(sizeof(uint2), sizeof(build_stage<ENS_BUILD_SPLIT>)) <= BUILD_LDS, "");
 template <bool MULTI>

@@ -387,8 +387,8 @@ __global__ __launch_bounds__(256) void pair_force_split_kernel(
 //    the list of each of its `active` particles is split into k = 64 / active
 //    (at most SPLIT_MAX) runs of whole blocks, one lane each, and lane p adds
 //    the runs of lanes p + active, p + 2 active, ... in that order (Kahan).
-//    One pass over the list: at N = 2^20, where issue is the bound, 96 us
-//    against 103 us with streams (equal below 2^18).
+//    One pass over the list: at N = 2^20, where issue is the bound, 97 us
+//    against 104 us with streams (within 5% of them below 2^18).
 // One cell segment of the staged force: the whole workgroup calls it for the
 // segment `seg` of the system described by (posq, off, sp, list, count, cap,
 // P); shared by the single-system kernel and the ensemble kernel.

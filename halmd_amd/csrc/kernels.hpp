@@ -373,9 +373,11 @@ struct displacement_check {
 constexpr unsigned PUBLISH_RING = 4;
 
 // Systems below FORCE_STREAMS_BELOW particles sum each particle's force in two
-// streams (force.hip), a result that does not depend on the segment shape;
-// larger ones in one pass: equal at N = 256,000 (35 us), 53 against 51 us at
-// N = 524,288, 102 against 93 us at N = 2^20.
+// streams (force.hip), a result that does not depend on the segment shape, so
+// that the shape can follow the system; larger ones, whose shape does not need
+// to, in one pass.  Streams against one pass, in us: 20.9 and 20.1 at N = 100,000,
+// 42.6 and 43.3 at 256,000 (two species), 30.4 and 29.8 at 262,143, 53.5 and 51.9
+// at 524,288, 104 and 97 at 2^20, 204 and 183 at 2^21.
 constexpr unsigned FORCE_STREAMS_BELOW = 1u << 18;
 __host__ __device__ inline bool force_streams(unsigned n) { return n < FORCE_STREAMS_BELOW; }
 // the same over 16-bit slot lists of cell segments (particles in cell order);
