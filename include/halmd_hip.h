@@ -256,7 +256,8 @@ HALMD_API int halmd_mdsim_neighbours_from_binning_entry_bytes(const halmd_neighb
 HALMD_API int halmd_mdsim_neighbours_from_binning_segments(const halmd_neighbour* nb, unsigned* cells,
                                                            unsigned* rows, unsigned* threads);
 /* sets the cell-segment shape (clamped to the grid; threads a multiple of 64,
- * at most 256) and rebuilds the lists at their next use; ignored for
+ * at most 256: of the force kernel, and of the list build by one lane for each
+ * particle) and rebuilds the lists at their next use; ignored for
  * global-index lists.  No counterpart in the reference (its from_binning
  * tuning knobs are the algorithm and unroll options, from_binning.cpp:328-339) */
 HALMD_API int halmd_mdsim_neighbours_from_binning_set_segments(halmd_neighbour* nb, unsigned cells, unsigned rows,
